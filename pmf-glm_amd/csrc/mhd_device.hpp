@@ -6,7 +6,7 @@
 // between the terms that divide by the same quantity, and the four-way HLLD flux choice
 // is a select between the left and right star fans rather than four flux evaluations.
 // Float kernels use the hardware v_rcp_f32 / v_sqrt_f32 / v_rsq_f32 (about 1 ulp);
-// double kernels use exact division and square root.
+// double kernels refine the hardware estimates to double precision.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -22,6 +22,7 @@ template <class T> struct StepParams {
   T gamma, gm1, igm1;        // gamma, gamma-1, 1/(gamma-1)
   T smallr, pfl, llf_dmin, llf_pmin;
   T ch, ich, ch2;            // GLM speed, 1/ch, ch^2 (ch = 0 for CT: ich unused)
+  T hch, hich;               // ch/2, 1/(2 ch)
   T dtdx, hdtdx, decay;      // dt/dx, dt/(2dx), psi factor
   int32_t recon, rsolve;
 };
@@ -39,11 +40,35 @@ struct Grid {
 };
 
 __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
-__device__ __forceinline__ double rcp(double x) { return 1.0 / x; }
+// Double: the hardware estimates (about 2^-23) refined with FMAs. A correctly rounded
+// division costs eleven instructions and a square root fourteen; the reciprocal below is
+// six and the roots eight and seven, with the last step a single-rounded FMA, so they are
+// within a rounding of the exact quotient and root (zero and infinity as for 1/x, sqrt). With
+// the HLLD form below a float64 160^3 MonCen step went from 800 to 708 us, its distance from a
+// 64-bit evaluation of the scheme unchanged (8e-17 of the state).
+__device__ __forceinline__ double rcp(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+  r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+  return __builtin_amdgcn_div_fixup(r, x, 1.0);
+}
 __device__ __forceinline__ float dsqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
-__device__ __forceinline__ double dsqrt(double x) { return __builtin_sqrt(x); }
+__device__ __forceinline__ double dsqrt(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = __builtin_fma(-h, g, 0.5);
+  g = __builtin_fma(g, r, g);
+  h = __builtin_fma(h, r, h);
+  g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  return __builtin_amdgcn_class(x, 0x260) ? x : g;  // +-0, +inf
+}
 __device__ __forceinline__ float rsq(float x) { return __builtin_amdgcn_rsqf(x); }
-__device__ __forceinline__ double rsq(double x) { return 1.0 / __builtin_sqrt(x); }
+__device__ __forceinline__ double rsq(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = __builtin_fma(-(x * y), y, 1.0);
+  const double r = __builtin_fma(y * e, __builtin_fma(0.375, e, 0.5), y);
+  return __builtin_amdgcn_class(x, 0x260) ? y : r;
+}
 __device__ __forceinline__ float dmax(float a, float b) { return __builtin_fmaxf(a, b); }
 __device__ __forceinline__ double dmax(double a, double b) { return __builtin_fmax(a, b); }
 __device__ __forceinline__ float dmin(float a, float b) { return __builtin_fminf(a, b); }
@@ -51,6 +76,8 @@ __device__ __forceinline__ double dmin(double a, double b) { return __builtin_fm
 __device__ __forceinline__ float dabs(float a) { return __builtin_fabsf(a); }
 __device__ __forceinline__ float dfma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double dfma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float dcopysign(float a, float b) { return __builtin_copysignf(a, b); }
+__device__ __forceinline__ double dcopysign(double a, double b) { return __builtin_copysign(a, b); }
 __device__ __forceinline__ double dabs(double a) { return __builtin_fabs(a); }
 
 // cons2prim (glm_physics.jl:11-18): density floored before the velocity and kinetic
@@ -195,37 +222,26 @@ __device__ __forceinline__ void hancock_plm(const T* m0, const T* dRx, const T* 
   for (int v = 0; v < 9; ++v) uh[v] = dfma(-P.dtdx, acc[v], uh[v]);
 }
 
+// The median of (a, b, 0).
+__device__ __forceinline__ float med3z(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, 0.f); }
+__device__ __forceinline__ double med3z(double a, double b) { return dmax(dmin(a, b), dmin(dmax(a, b), 0.0)); }
+
 // PLM face offsets (dL, dR) from the one-sided differences dl = q0 - qm and dr = qp - q0
 // (glm_physics.jl:47-59), for offsets<RECON> and for callers that already hold a
 // difference (the fused step carries each column's z difference from one plane to the
 // next).
 template <int RECON, class T> __device__ __forceinline__ void offsets_diff(T dl, T dr, T& dL, T& dR) {
   static_assert(RECON != RECON_PPM, "PLM only");
-  if constexpr (sizeof(T) == 4) {
-    // minmod(a, b) is the median of (a, b, 0), and MonCen the median of (2 minmod(a, b),
-    // (a+b)/2, 0): one v_med3_f32 each instead of the sign/abs/min/compare chain (equal
-    // to glm_physics.jl's form except where a*b underflows to zero)
-    T mm = __builtin_amdgcn_fmed3f(dl, dr, T(0));
-    T s;
-    if constexpr (RECON == RECON_PLM_MINMOD) s = mm;
-    else s = __builtin_amdgcn_fmed3f(T(2) * mm, T(0.5) * (dl + dr), T(0));
-    s = T(0.5) * s;
-    dL = -s;
-    dR = s;
-  } else {
-    T s;
-    if constexpr (RECON == RECON_PLM_MINMOD) {
-      T m = dmin(dabs(dl), dabs(dr));
-      s = dl >= T(0) ? m : -m;
-    } else {
-      T dc = T(0.5) * (dl + dr);
-      T m = dmin(T(2) * dmin(dabs(dl), dabs(dr)), dabs(dc));
-      s = dc >= T(0) ? m : -m;
-    }
-    s = dl * dr <= T(0) ? T(0) : T(0.5) * s;
-    dL = -s;
-    dR = s;
-  }
+  // minmod(a, b) is the median of (a, b, 0), and half of MonCen the median of (minmod(a, b),
+  // (a+b)/4, 0) (powers of two scale exactly): one v_med3_f32 each, or four v_min/v_max_f64,
+  // instead of the sign/abs/min/compare chain (equal to glm_physics.jl's form except where
+  // a*b underflows to zero)
+  const T mm = med3z(dl, dr);
+  T s;
+  if constexpr (RECON == RECON_PLM_MINMOD) s = T(0.5) * mm;
+  else s = med3z(mm, T(0.25) * (dl + dr));
+  dL = -s;
+  dR = s;
 }
 
 // Limited face offsets (dL, dR) of one primitive from its two neighbours
@@ -242,15 +258,8 @@ template <int RECON, class T> __device__ __forceinline__ void offsets(T qm, T q0
     T slope = (qp - qm) * T(0.25);
     T curve = (qm - T(2) * q0 + qp) * T(1.0 / 12.0);
     T a = slope + curve, b = slope - curve;
-    if constexpr (sizeof(T) == 4) {
-      dR = __builtin_amdgcn_fmed3f(a, T(2) * b, T(0));
-      dL = -__builtin_amdgcn_fmed3f(b, T(2) * a, T(0));
-    } else {
-      const bool flat = a * b <= T(0);
-      const T a2 = T(2) * a, b2 = T(2) * b;
-      dR = flat ? T(0) : (dabs(a) > dabs(b2) ? b2 : a);
-      dL = flat ? T(0) : -(dabs(b) > dabs(a2) ? a2 : b);
-    }
+    dR = med3z(a, T(2) * b);
+    dL = -med3z(b, T(2) * a);
   } else {
     offsets_diff<RECON>(q0 - qm, qp - q0, dL, dR);
   }
@@ -349,9 +358,11 @@ __device__ __forceinline__ void hll_n(const T* L, const T* R, T bn, T fbn, T fps
 // HLLD (Miyoshi & Kusano 2005) as in glm_physics.jl:255-307. The flux is
 //   F_side + S*(U*_side - U_side) + [inner]*S*_side*(U**_side - U*_side)
 // with side = left when SM >= 0 and "inner" the two branches that use the double-star
-// state; this equals the reference's four formulas branch by branch.
+// state; this equals the reference's four formulas branch by branch, with their guards: the
+// star-density floor and the degenerate star states. hlld_n takes it for the faces whose
+// guards act.
 template <class T>
-__device__ __forceinline__ void hlld_n(const T* L, const T* R, T bn, T fbn, T fpsi, T* f, const StepParams<T>& P) {
+__device__ __forceinline__ void hlld_guarded_n(const T* L, const T* R, T bn, T fbn, T fpsi, T* f, const StepParams<T>& P) {
   const T dL = L[0], uL = L[1], vL = L[2], wL = L[3], pL = L[4], byL = L[6], bzL = L[7];
   const T dR = R[0], uR = R[1], vR = R[2], wR = R[3], pR = R[4], byR = R[6], bzR = R[7];
   const T bn2 = bn * bn;
@@ -439,6 +450,94 @@ __device__ __forceinline__ void hlld_n(const T* L, const T* R, T bn, T fbn, T fp
   f[8] = fpsi;
 }
 
+// HLLD on the faces where no guard acts (all but pathological ones). There each state of the
+// fan obeys the jump conditions with its neighbour exactly: the flux of the state U that
+// holds at the face (U* of the side of SM, or U** inside the Alfven waves) is
+//   rho* SM, rho* SM^2 + pt* - bn^2, rho* SM v - bn b, (E + pt*) SM - bn v.B, SM b - bn v
+// with that state's v, b and E, and equals F_side + S (U* - U_side) [+ S* (U** - U*)] of
+// hlld_guarded_n. So the outer states enter through E* only, U** is U* plus the Alfven jump
+// (db = sign(bn) sqrt(rho*) dv), pt* comes from the selected side, and the two fast speeds
+// share their outer root. The fused step is bound by VALU issue (0.96 of the peak rate): about
+// 220 issue slots per face instead of 275 took two 256^3 minmod steps from 1694 to 1610 us, a
+// 512^3 step from 6.80 to 6.56 ms, a 128^3 PPM step from 110 to 105 us. A face with a floored star
+// density or a degenerate star state (found from values this path needs anyway) goes to
+// hlld_guarded_n, in a branch that no wave of an ordinary flow takes. Pinned (explicit FMAs
+// only): every kernel that inlines it gives the same bits.
+template <class T>
+__device__ __forceinline__ void hlld_n(const T* L, const T* R, T bn, T fbn, T fpsi, T* f, const StepParams<T>& P) {
+#pragma clang fp contract(off)
+  const T dL = L[0], uL = L[1], vL = L[2], wL = L[3], pL = L[4], byL = L[6], bzL = L[7];
+  const T dR = R[0], uR = R[1], vR = R[2], wR = R[3], pR = R[4], byR = R[6], bzR = R[7];
+  const T bn2 = bn * bn, bn4 = T(4) * bn2;
+  const T irL = rcp(dL), irR = rcp(dR);
+  const T b2L = dfma(bzL, bzL, dfma(byL, byL, bn2)), b2R = dfma(bzR, bzR, dfma(byR, byR, bn2));
+  const T ptL = dfma(T(0.5), b2L, pL), ptR = dfma(T(0.5), b2R, pR);
+  // c_fast^2 = (s + sqrt(s^2 - 4 c^2 bn^2/rho)) / 2 with s = c^2 + |B|^2/rho
+  const T c2L = (P.gamma * pL) * irL, c2R = (P.gamma * pR) * irR;
+  const T sL = dfma(b2L, irL, c2L), sR = dfma(b2R, irR, c2R);
+  const T qL = sL + dsqrt(dmax(dfma(sL, sL, -(c2L * (bn4 * irL))), T(0)));
+  const T qR = sR + dsqrt(dmax(dfma(sR, sR, -(c2R * (bn4 * irR))), T(0)));
+  const T cmax = dsqrt(T(0.5) * dmax(qL, qR));
+  const T SL = dmin(dmin(uL, uR) - cmax, T(0));
+  const T SR = dmax(dmax(uL, uR) + cmax, T(0));
+  const T oL = SL - uL, oR = SR - uR;
+  const T aL = oL * dL, aR = oR * dR;  // mass fluxes relative to the outer waves
+  const T SM = dfma(aR, uR, dfma(-aL, uL, ptL - ptR)) * rcp(aR - aL);
+  const T eL = SL - SM, eR = SR - SM;
+  const T iLM = rcp(eL), iRM = rcp(eR);
+  const T dLs = aL * iLM, dRs = aR * iRM;
+  const T kL = dfma(aL, eL, -bn2), kR = dfma(aR, eR, -bn2);
+  const bool guarded = !(dLs >= T(1e-12)) || !(dRs >= T(1e-12)) || dabs(kL) < T(1e-12) || dabs(kR) < T(1e-12);
+  if (__builtin_expect(guarded, 0)) {
+    hlld_guarded_n(L, R, bn, fbn, fpsi, f, P);
+    return;
+  }
+  const T rqL = rsq(dLs), rqR = rsq(dRs);
+  const T sqL = dLs * rqL, sqR = dRs * rqR;
+  // single-star transverse states (glm_physics.jl:255-263)
+  const T ikL = rcp(kL), ikR = rcp(kR);
+  const T fcL = (bn * (SM - uL)) * ikL, fcR = (bn * (SM - uR)) * ikR;
+  const T ggL = dfma(aL, oL, -bn2) * ikL, ggR = dfma(aR, oR, -bn2) * ikR;
+  const T vyLs = dfma(-byL, fcL, vL), vzLs = dfma(-bzL, fcL, wL), byLs = byL * ggL, bzLs = bzL * ggL;
+  const T vyRs = dfma(-byR, fcR, vR), vzRs = dfma(-bzR, fcR, wR), byRs = byR * ggR, bzRs = bzR * ggR;
+  // double-star state (glm_physics.jl:288-296) as the left star plus its Alfven jump
+  const T sg = dcopysign(T(1), bn);
+  const T isum = rcp(sqL + sqR);
+  const T jy = dfma(sqR, vyRs - vyLs, sg * (byRs - byLs)) * isum;
+  const T jz = dfma(sqR, vzRs - vzLs, sg * (bzRs - bzLs)) * isum;
+  const T sgL = sg * sqL;
+  const T vyss = vyLs + jy, vzss = vzLs + jz;
+  const T byss = dfma(sgL, jy, byLs), bzss = dfma(sgL, jz, bzLs);
+  const T SMbn = SM * bn;
+  const T vbss = dfma(vzss, bzss, dfma(vyss, byss, SMbn));
+  // the side of the contact (glm_physics.jl:297-305)
+  const bool left = SM >= T(0);
+  const T d = left ? dL : dR, u = left ? uL : uR, v = left ? vL : vR, w = left ? wL : wR;
+  const T p = left ? pL : pR, by = left ? byL : byR, bz = left ? bzL : bzR, pt = left ? ptL : ptR;
+  const T o = left ? oL : oR, iM = left ? iLM : iRM, ds = left ? dLs : dRs, sq = left ? sqL : sqR;
+  const T vys = left ? vyLs : vyRs, vzs = left ? vzLs : vzRs, bys = left ? byLs : byRs, bzs = left ? bzLs : bzRs;
+  const T pts = dfma(o * d, SM - u, pt);
+  const T E = dfma(T(0.5) * d, dfma(w, w, dfma(v, v, u * u)), dfma(p, P.igm1 - T(1), pt));
+  const T vb = dfma(w, bz, dfma(v, by, u * bn));
+  const T vbs = dfma(vzs, bzs, dfma(vys, bys, SMbn));
+  const T Es = dfma(-bn, vbs, dfma(pts, SM, dfma(bn, vb, dfma(-pt, u, o * E)))) * iM;
+  const T abn = dabs(bn);
+  const bool inner = left ? dfma(-abn, rqL, SM) < T(0) : dfma(abn, rqR, SM) >= T(0);
+  const T vy = inner ? vyss : vys, vz = inner ? vzss : vzs, fy = inner ? byss : bys, fz = inner ? bzss : bzs;
+  const T vbx = inner ? vbss : vbs;
+  const T Ex = dfma(sq * (left ? -sg : sg), vbs - vbx, Es);
+  const T m = ds * SM;
+  f[0] = m;
+  f[1] = dfma(m, SM, pts - bn2);
+  f[2] = dfma(m, vy, -(bn * fy));
+  f[3] = dfma(m, vz, -(bn * fz));
+  f[4] = dfma(Ex + pts, SM, -(bn * vbx));
+  f[5] = fbn;
+  f[6] = dfma(SM, fy, -(bn * vy));
+  f[7] = dfma(SM, fz, -(bn * vz));
+  f[8] = fpsi;
+}
+
 // riemann / riemann_ct (glm_physics.jl:317-348) on normal-frame states (modified in place:
 // floors, and the normal field replaced by the GLM b_n*, or by the CT face value).
 template <bool CT, class T, int RS = -1>
@@ -459,8 +558,9 @@ __device__ __forceinline__ void riemann_n(T* L, T* R, T* f, const StepParams<T>&
     // product, and a caller's flux difference F_lo - F_hi could otherwise fuse one face's
     // product into an FMA, so that equal fluxes would not cancel
 #pragma clang fp contract(off)
-    bns = T(0.5) * (L[5] + R[5]) - T(0.5) * (R[8] - L[8]) * P.ich;
-    fbn = T(0.5) * (L[8] + R[8]) - T(0.5) * P.ch * (R[5] - L[5]);
+    // (the FMAs' products by 1/2 are exact, so they round as the separate operations do)
+    bns = dfma(T(0.5), L[5] + R[5], -((R[8] - L[8]) * P.hich));
+    fbn = dfma(T(0.5), L[8] + R[8], -(P.hch * (R[5] - L[5])));
     fpsi = P.ch2 * bns;
     ch = P.ch;
   }
@@ -475,6 +575,8 @@ __device__ __forceinline__ void riemann_n(T* L, T* R, T* f, const StepParams<T>&
                  (P.llf_pmin > T(0) && dmin(L[4], R[4]) < P.llf_pmin);
     if (uself)
       llf_n(L, R, ch, fbn, fpsi, f, P);
+    else if constexpr (CT)  // its GS05 upwinding switches on the sign of the mass flux, so the form is kept
+      hlld_guarded_n(L, R, bns, fbn, fpsi, f, P);
     else
       hlld_n(L, R, bns, fbn, fpsi, f, P);
   }

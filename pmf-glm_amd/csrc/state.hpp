@@ -114,6 +114,8 @@ template <class T> StepParams<T> make_params(const pmf_state* s, double dt, doub
   P.ch = T(ch);
   P.ich = ch != 0.0 ? T(1) / T(ch) : T(0);
   P.ch2 = T(ch) * T(ch);
+  P.hch = T(0.5) * P.ch;
+  P.hich = T(0.5) * P.ich;
   P.dtdx = T(dt) / T(p.dx);
   P.hdtdx = T(0.5) * P.dtdx;
   P.decay = T(decay);

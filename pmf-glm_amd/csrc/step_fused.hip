@@ -1015,6 +1015,8 @@ __global__ __launch_bounds__(64) void k_step_params(const double* __restrict__ d
   P.ch = T(ch);
   P.ich = ch != 0.0 ? T(1) / T(ch) : T(0);
   P.ch2 = T(ch) * T(ch);
+  P.hch = T(0.5) * P.ch;
+  P.hich = T(0.5) * P.ich;
   P.dtdx = T(dtf) / T(dx);
   P.hdtdx = T(0.5) * P.dtdx;
   P.decay = T(decay);
@@ -1219,6 +1221,8 @@ __global__ __launch_bounds__(256) void k_ens_params(const EnsCube* __restrict__ 
     P.ch = chf;
     P.ich = chf != 0.f ? 1.f / chf : 0.f;
     P.ch2 = chf * chf;
+    P.hch = 0.5f * P.ch;
+    P.hich = 0.5f * P.ich;
     P.dtdx = float(dtf) / dxf;
     P.hdtdx = 0.5f * P.dtdx;
     const float v = -cr * chf * float(dtf) / dxf;

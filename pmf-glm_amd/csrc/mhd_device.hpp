@@ -464,7 +464,8 @@ __device__ __forceinline__ void hlld_guarded_n(const T* L, const T* R, T bn, T f
 // hlld_guarded_n, in a branch that no wave of an ordinary flow takes. Pinned (explicit FMAs
 // only): every kernel that inlines it gives the same bits.
 template <class T>
-__device__ __forceinline__ void hlld_n(const T* L, const T* R, T bn, T fbn, T fpsi, T* f, const StepParams<T>& P) {
+__device__ __forceinline__ void hlld_n(const T* L, const T* R, T bn, T fbn, T fpsi, T* f, const StepParams<T>& P,
+                                       bool llf = false) {
 #pragma clang fp contract(off)
   const T dL = L[0], uL = L[1], vL = L[2], wL = L[3], pL = L[4], byL = L[6], bzL = L[7];
   const T dR = R[0], uR = R[1], vR = R[2], wR = R[3], pR = R[4], byR = R[6], bzR = R[7];
@@ -487,9 +488,10 @@ __device__ __forceinline__ void hlld_n(const T* L, const T* R, T bn, T fbn, T fp
   const T iLM = rcp(eL), iRM = rcp(eR);
   const T dLs = aL * iLM, dRs = aR * iRM;
   const T kL = dfma(aL, eL, -bn2), kR = dfma(aR, eR, -bn2);
-  const bool guarded = !(dLs >= T(1e-12)) || !(dRs >= T(1e-12)) || dabs(kL) < T(1e-12) || dabs(kR) < T(1e-12);
+  const bool guarded = llf || !(dLs >= T(1e-12)) || !(dRs >= T(1e-12)) || dabs(kL) < T(1e-12) || dabs(kR) < T(1e-12);
   if (__builtin_expect(guarded, 0)) {
-    hlld_guarded_n(L, R, bn, fbn, fpsi, f, P);
+    if (llf) llf_n(L, R, P.ch, fbn, fpsi, f, P);
+    else hlld_guarded_n(L, R, bn, fbn, fpsi, f, P);
     return;
   }
   const T rqL = rsq(dLs), rqR = rsq(dRs);
@@ -573,12 +575,15 @@ __device__ __forceinline__ void riemann_n(T* L, T* R, T* f, const StepParams<T>&
   } else {
     bool uself = (P.llf_dmin > T(0) && dmin(L[0], R[0]) < P.llf_dmin) ||
                  (P.llf_pmin > T(0) && dmin(L[4], R[4]) < P.llf_pmin);
-    if (uself)
-      llf_n(L, R, ch, fbn, fpsi, f, P);
-    else if constexpr (CT)  // its GS05 upwinding switches on the sign of the mass flux, so the form is kept
-      hlld_guarded_n(L, R, bns, fbn, fpsi, f, P);
-    else
-      hlld_n(L, R, bns, fbn, fpsi, f, P);
+    if constexpr (CT) {
+      // its GS05 upwinding switches on the sign of the mass flux, so the form is kept
+      if (uself)
+        llf_n(L, R, ch, fbn, fpsi, f, P);
+      else
+        hlld_guarded_n(L, R, bns, fbn, fpsi, f, P);
+    } else {
+      hlld_n(L, R, bns, fbn, fpsi, f, P, uself);
+    }
   }
 }
 

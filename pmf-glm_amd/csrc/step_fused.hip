@@ -9,7 +9,8 @@
 // m and m-1 with both halo rings; the next plane enters the buffer of m-1 as soon as
 // each column's own slot there is no longer needed. With the kernel's register budget
 // (about 165 VGPRs) a SIMD holds three waves for the float minmod and MonCen-HLL/LLF
-// variants (two for the rest), so three (two) 4-wave workgroups share a CU. Per plane m:
+// variants (two for the rest, float64 PLM among them), so three (two) 4-wave workgroups
+// share a CU. Per plane m:
 //   1. convert the next plane of the own column (and, for a few threads, of the extra
 //      halo cells) from conserved to primitive;
 //   2. Hancock-predict plane m in every column (cons2prim of the half-step state);
@@ -408,9 +409,10 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
 
   static_assert(!(SRC && SURR), "the surrogate path has no source terms");
   bool mkz = false, mkzp = false;  // masked-fallback flags of this column's planes m and m-1
-  // PLM without source terms: this column's z difference q(m) - q(m-1), carried from
-  // plane to plane (the source and surrogate variants, short of registers, re-read it)
-  constexpr bool ZCARRY = RECON != RECON_PPM && !SRC && !SURR;
+  // float PLM without source terms: this column's z difference q(m) - q(m-1), carried from
+  // plane to plane (the source, surrogate and float64 variants, short of registers, re-read
+  // it)
+  constexpr bool ZCARRY = RECON != RECON_PPM && !SRC && !SURR && sizeof(T) == 4;
   T dzc[9];
   for (int m = z0 - 1; m <= z0 + zc; ++m) {
     const bool first = m == z0 - 1, last = m == z0 + zc;
@@ -865,10 +867,20 @@ __device__ __forceinline__ void block_store_max(T smax, T* sMax, double* out) {
 // spilling; PPM keeps both edge offsets of each direction live and is still faster at
 // three waves than at two. The PLM source variants (drag, radiation) spill 4-7 dwords at
 // three waves and run 14-17% faster than at two; the PPM source variants would spill 44
-// and keep the compiler's default (two waves), as do the surrogate and float64 variants.
+// and keep the compiler's default (two waves).
 template <class T, int RECON, int RS, bool SURR, bool SRC>
 constexpr bool fused_three_waves() {
   return sizeof(T) == 4 && !SURR && !(SRC && RECON == RECON_PPM);
+}
+
+// Two waves per SIMD (256 registers): the surrogate step, and float64 PLM, whose plain
+// variants the compiler would otherwise give 280-320 registers and one wave, which leaves
+// every dependent FMA waiting for its result (160^3: HLLD 708 -> 612 us although 27 dwords
+// spill there, HLL, without spills, 649 -> 429). PPM would spill 61 and stays at one wave
+// (762 us against 901), with its divergence carry in LDS; so do the source variants.
+template <class T, int RECON, bool SURR, bool SRC>
+constexpr bool fused_two_waves() {
+  return SURR || (sizeof(T) == 8 && !SRC && RECON != RECON_PPM);
 }
 
 // The single-grid step: one workgroup per work item. simg is the network's image in
@@ -930,14 +942,16 @@ __global__ __launch_bounds__(FTHREADS) __attribute__((amdgpu_waves_per_eu(3))) v
   step_fused_body<T, RECON, RS, SURR, SRC, NARROW, BCG>(U, O, g, P, red, simg, thr, nsmooth, src);
 }
 
-// The surrogate-assisted step: two waves per SIMD (about 250 VGPRs with the network in its
-// own function; 81.6 KB of LDS), so two workgroups share a CU and one's network batches
-// overlap the other's HLLD faces and barriers.
-template <class T, int RECON, int RS, bool SURR, bool SRC, bool NARROW>
+// Two waves per SIMD. The surrogate-assisted step: about 250 VGPRs with the network in its
+// own function and 81.6 KB of LDS, so two workgroups share a CU and one's network batches
+// overlap the other's HLLD faces and barriers. float64 PLM: 76 KB of LDS, two workgroups.
+template <class T, int RECON, int RS, bool SURR, bool SRC, bool NARROW, bool BCG>
 __global__ __launch_bounds__(FTHREADS) __attribute__((amdgpu_waves_per_eu(2))) void k_step_fused2(
-    Fields<const T> U, Fields<T> O, FusedGeom g, StepParams<T> P, double* __restrict__ red,
-    const unsigned char* __restrict__ simg, float thr, unsigned long long* __restrict__ nsmooth, SrcParams<T> src) {
-  step_fused_body<T, RECON, RS, SURR, SRC, NARROW>(U, O, g, P, red, simg, thr, nsmooth, src);
+    Fields<const T> U, Fields<T> O, FusedGeom g, StepParams<T> P, const StepParams<T>* __restrict__ Pd,
+    double* __restrict__ red, const unsigned char* __restrict__ simg, float thr,
+    unsigned long long* __restrict__ nsmooth, SrcParams<T> src) {
+  if (Pd) P = *Pd;
+  step_fused_body<T, RECON, RS, SURR, SRC, NARROW, BCG>(U, O, g, P, red, simg, thr, nsmooth, src);
 }
 
 template <class T, int RECON, int RS, bool SURR, bool SRC = false, bool NARROW = false, bool BCG = false>
@@ -948,9 +962,9 @@ void launch_fused_variant(dim3 grd, hipStream_t st, const Fields<const T>& U, co
   if constexpr (fused_three_waves<T, RECON, RS, SURR, SRC>())
     hipLaunchKernelGGL((k_step_fused3<T, RECON, RS, SURR, SRC, NARROW, BCG>), grd, dim3(FTHREADS), 0, st, U, O, g, P,
                        Pd, red, simg, thr, nsmooth, src);
-  else if constexpr (SURR)
-    hipLaunchKernelGGL((k_step_fused2<T, RECON, RS, SURR, SRC, NARROW>), grd, dim3(FTHREADS), 0, st, U, O, g, P, red,
-                       simg, thr, nsmooth, src);
+  else if constexpr (fused_two_waves<T, RECON, SURR, SRC>())
+    hipLaunchKernelGGL((k_step_fused2<T, RECON, RS, SURR, SRC, NARROW, BCG>), grd, dim3(FTHREADS), 0, st, U, O, g, P,
+                       Pd, red, simg, thr, nsmooth, src);
   else
     hipLaunchKernelGGL((k_step_fused<T, RECON, RS, SURR, SRC, NARROW, BCG>), grd, dim3(FTHREADS), 0, st, U, O, g, P,
                        Pd, red, simg, thr, nsmooth, src);

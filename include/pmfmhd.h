@@ -153,7 +153,8 @@ int pmf_set_chunk(pmf_state* s, int32_t zc);
 /* Times the fused kernel (the plain step, or the fused CT step for CT states) for z
  * chunks of 4..128 planes (reps launches each, writing only the scratch fields and, for
  * CT, the per-step workspace slots) and keeps the fastest; returns it and its time per
- * step. */
+ * step. Small grids whose built-in choice is shorter than 4 planes keep that one if it is
+ * faster; the depth returned is then the fastest of 4..128. */
 int pmf_autotune(pmf_state* s, int32_t reps, int32_t* zc_out, double* ms_out);
 /* Kernel of the CT (:ref) step. By default a constrained-transport state steps (plain,
  * drag and radiation steps alike) on the fused z-marching kernel, which solves every face

@@ -295,7 +295,9 @@ void create_state(const pmf_params* pp, pmf_state** out, bool with_fields) {
         hip_check(hipMemsetAsync(s->ct, 0, 21 * s->nc * s->esz, s->st), "hipMemset");
       }
     }
-    size_t nred = std::max<size_t>(size_t(kRedBlocks) * kRedSlots, size_t(fused_blocks(s->G, kMinChunk)));
+    const bool f64 = p.precision == PMF_F64;
+    const size_t nred = std::max<size_t>(size_t(kRedBlocks) * kRedSlots,
+                                         size_t(std::max(fused_blocks(s->G, f64), fused_blocks(s->G, f64, kMinChunk))));
     hip_check(hipMalloc(&s->red, sizeof(double) * nred), "hipMalloc(red)");
     hip_check(hipMalloc(&s->dval, sizeof(double) * 64), "hipMalloc(dval)");
     hip_check(hipHostMalloc((void**)&s->hval, sizeof(double) * 64, hipHostMallocDefault), "hipHostMalloc");
@@ -582,11 +584,15 @@ int pmf_autotune(pmf_state* s, int32_t reps, int32_t* zc_out, double* ms_out) {
     hip_check(hipEventCreate(&e0), "hipEventCreate");
     hip_check(hipEventCreate(&e1), "hipEventCreate");
     const int keep = s->zc;
-    int best_zc = 0;
-    double best = 1e300;
+    int best_zc = 0, keep_zc = 0;
+    double best = 1e300, best_set = 1e300;
     try {
-      for (int zc : {4, 8, 12, 16, 24, 32, 48, 64, 96, 128}) {
-        if (zc > s->G.nz && zc != 4) break;
+      // the built-in choice (0) too, where it is shorter than any depth a caller may set: it is
+      // kept if it is the fastest, and the depth returned is then the fastest settable one
+      const int first = fused_chunk(s->G, s->p.precision == PMF_F64) < kMinChunk ? 0 : 4;
+      for (int zc : {0, 4, 8, 12, 16, 24, 32, 48, 64, 96, 128}) {
+        if (zc < first) continue;
+        if (zc > s->G.nz && zc > 4) break;
         s->zc = zc;
         // writes only the scratch fields (and, for CT, workspace slots 3-14 or the edge
         // EMFs 15-17, which every step recomputes): the state and its CT faces are untouched
@@ -616,6 +622,10 @@ int pmf_autotune(pmf_state* s, int32_t reps, int32_t* zc_out, double* ms_out) {
         hip_check(hipEventElapsedTime(&ms, e0, e1), "hipEventElapsedTime");
         if (ms / reps < best) {
           best = ms / reps;
+          keep_zc = zc;
+        }
+        if (zc > 0 && ms / reps < best_set) {
+          best_set = ms / reps;
           best_zc = zc;
         }
       }
@@ -627,7 +637,7 @@ int pmf_autotune(pmf_state* s, int32_t reps, int32_t* zc_out, double* ms_out) {
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    s->zc = best_zc;
+    s->zc = keep_zc;
     s->smax_valid = false;  // dval now holds the speed of the scratch fields
     if (zc_out) *zc_out = best_zc;
     if (ms_out) *ms_out = best;
@@ -859,7 +869,7 @@ double* static_workspace() {
 int64_t static_partials_needed(const pmf_params& p, int integrator, bool want_smax) {
   const int64_t nc = int64_t(p.nx) * p.ny * p.nz;
   const Grid G{p.nx, p.ny, p.nz, {p.bc[0], p.bc[1], p.bc[2]}, nc};
-  if (p.solver == PMF_SOLVER_GLM && integrator == PMF_INTEGRATOR_CUBE) return fused_blocks(G, 0);
+  if (p.solver == PMF_SOLVER_GLM && integrator == PMF_INTEGRATOR_CUBE) return fused_blocks(G, p.precision == PMF_F64);
   if (p.solver == PMF_SOLVER_CT || want_smax) return int64_t(kRedBlocks) * kRedSlots;
   return 0;
 }

@@ -53,10 +53,11 @@ bool launch_step_fused_ct(Fields<const T> U, Fields<T> O, T* ctp, const Grid& G,
 bool launch_step_fused_surr(Fields<const float> U, Fields<float> O, const Grid& G, const StepParams<float>& P,
                             double* red, double* dsmax, const unsigned char* simg, float thr,
                             unsigned long long* nsmooth, hipStream_t st);
-// Number of workgroups (one partial maximum each) the fused kernel launches for G with
-// z chunks of zc planes (0 = the built-in choice).
-int64_t fused_blocks(const Grid& G, int zc = 0);
-constexpr int kMinChunk = 4;  // smallest z chunk the library accepts
+// Number of workgroups (one partial maximum each) the fused kernel launches for G in the
+// given precision with z chunks of zc planes (0 = the built-in choice).
+int64_t fused_blocks(const Grid& G, bool f64, int zc = 0);
+int fused_chunk(const Grid& G, bool f64);  // the built-in z chunk
+constexpr int kMinChunk = 4;  // smallest z chunk a caller may set (the built-in choice may be shorter)
 
 // Geometry of the fused kernel's work decomposition: 16x12 column tiles (x fastest,
 // then y; the last tile row may be ragged) marched through z chunks of zc planes.

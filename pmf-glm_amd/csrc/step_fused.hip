@@ -847,6 +847,14 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
   return smax;
 }
 
+// XCD-aware tile order: dispatch round-robins workgroups over the 8 XCDs, so XCD x gets
+// workgroups x, x + 8, ...; they take a contiguous range of tiles (nwg / 8, one more for the
+// first nwg % 8 XCDs), whose halo re-reads its L2 then serves.
+__device__ __forceinline__ int xcd_tile() {
+  const int nwg = gridDim.x, x = blockIdx.x & 7;
+  return x * (nwg >> 3) + min(x, nwg & 7) + (blockIdx.x >> 3);
+}
+
 // Block-wide CFL maximum of the threads' running maxima, stored by thread 0.
 template <class T>
 __device__ __forceinline__ void block_store_max(T smax, T* sMax, double* out) {
@@ -900,11 +908,7 @@ __device__ __forceinline__ void step_fused_body(const Fields<const T>& U, const 
     unsigned* dw = reinterpret_cast<unsigned*>(sW);
     for (int e = threadIdx.x; e < SIMG_NW / 2; e += FTHREADS) dw[e] = src[e];
   }
-  // XCD-aware tile order: dispatch round-robins workgroups over the 8 XCDs, so
-  // logical tile (w % 8) * (nwg / 8) + w / 8 gives each XCD a contiguous tile range.
-  const int nwg = gridDim.x;
-  int w = blockIdx.x;
-  if ((nwg & 7) == 0) w = (w & 7) * (nwg >> 3) + (w >> 3);
+  const int w = xcd_tile();
   SurrQueue<FQCAP>* q = nullptr;
   if constexpr (SURR) q = &sQ;
   // the biases (the image's float tail) stay in global memory: with them out of LDS the
@@ -1057,8 +1061,8 @@ static FusedGeom fused_geom(const Grid& G, int zc) {
   g.nz = G.nz;
   g.ntx = (G.nx + TX - 1) / TX;
   g.nty = (G.ny + TY - 1) / TY;
-  g.zc = zc;
   g.nchunks = (G.nz + zc - 1) / zc;
+  g.zc = (G.nz + g.nchunks - 1) / g.nchunks;  // as many chunks, of equal length: no XCD gets only short ones
   g.plane = (int64_t)G.nx * G.ny;
   g.nc = G.nc;
   for (int d = 0; d < 3; ++d) g.bc[d] = G.bc[d];
@@ -1098,26 +1102,45 @@ static int device_cus() {
   return cus[dev];
 }
 
-// z-chunk length: long enough that the two extra prediction planes per chunk stay
-// small, short enough to give a few workgroups per CU. Halving from 32 until the grid
-// has at least 2048 workgroups suits large grids; on small ones it ends at 4-8 planes,
-// where a chunk of 16 whose workgroups fill most of one round (three per CU) wastes
-// fewer planes (128^3: 704 workgroups, 0.136 vs 0.153 ms at 4; at 160^3, 96^3 and 192^3
-// the halving rule's choice measured best).
-static int pick_zc(const Grid& G) {
+// z-chunk length. A chunk of zc planes costs about zc + 2 of them (two more planes are
+// predicted at its ends), and a CU that holds 1, 2 or 3 workgroups steps a plane of each
+// in 3.7, 4.4 or 5.7 us (float; float64, two a CU: 7.1, 10.3): one or two workgroups leave
+// the SIMDs waiting on dependent instructions. So the choice weighs short chunks that fill
+// the CUs against the planes they repeat: full rounds of `slots` workgroups per CU, then the
+// last, partly filled one. Chunks past 32 planes repeat under 6% and measured no faster (256^3
+// 32: 790 us, 64: 876; 512^3 5.93 and 6.06 ms).
+// Measured (minmod, step and fold, the earlier rule's choice -> this one's): 16^3 23.7 -> 12.9
+// us (4 planes -> 1), 32^3 23.7 -> 13.6 (1), 64^3 31.4 -> 28.6 (2), 96^3 64 -> 55 (6); 128^3 (16)
+// and 256^3 (32) as before.
+static int pick_zc(const Grid& G, int slots) {
+  static const double kShare[2][4] = {{0, 1.0, 1.45, 1.45}, {0, 1.0, 1.19, 1.54}};
+  const double* share = kShare[slots >= 3];
   const int64_t tiles = (int64_t)((G.nx + TX - 1) / TX) * ((G.ny + TY - 1) / TY);
-  auto groups = [&](int zc) { return tiles * ((G.nz + zc - 1) / zc); };
-  int zc = 32;
-  while (zc > 4 && groups(zc) < 2048) zc >>= 1;
-  const int64_t round = 3 * (int64_t)device_cus();
-  if (zc <= 8 && groups(16) <= round && 3 * groups(16) >= 2 * round) zc = 16;
-  return zc < G.nz ? zc : G.nz;
+  const int64_t cus = device_cus();
+  int best = 1;
+  double cost = 1e300;
+  for (int zc = 1; zc <= 32 && zc <= G.nz; ++zc) {
+    const int chunks = (G.nz + zc - 1) / zc;
+    if (zc > 1 && (G.nz + chunks - 1) / chunks != zc) continue;  // a shorter chunk gives as many
+    const int64_t groups = tiles * chunks, full = groups / (slots * cus), rest = groups - full * slots * cus;
+    const double c = (double(full) * share[slots] + share[(rest + cus - 1) / cus]) * (zc + 2);
+    if (c < cost) {
+      cost = c;
+      best = zc;
+    }
+  }
+  return best;
 }
 
-static int chunk_of(const Grid& G, int zc) { return zc > 0 ? (zc < G.nz ? zc : G.nz) : pick_zc(G); }
+// Workgroups per CU of the fused step by precision (three float, two float64).
+static int chunk_of(const Grid& G, int zc, bool f64) {
+  return zc > 0 ? (zc < G.nz ? zc : G.nz) : pick_zc(G, f64 ? 2 : 3);
+}
 
-int64_t fused_blocks(const Grid& G, int zc) {
-  FusedGeom g = fused_geom(G, chunk_of(G, zc));
+int fused_chunk(const Grid& G, bool f64) { return chunk_of(G, 0, f64); }
+
+int64_t fused_blocks(const Grid& G, bool f64, int zc) {
+  FusedGeom g = fused_geom(G, chunk_of(G, zc, f64));
   return (int64_t)g.ntx * g.nty * g.nchunks;
 }
 
@@ -1125,7 +1148,7 @@ template <class T>
 bool launch_step_fused(Fields<const T> U, Fields<T> O, const Grid& G, const StepParams<T>& P, double* red,
                        double* dsmax, hipStream_t st, int zc, const SrcParams<T>* src, const StepParams<T>* Pd) {
   if (!fused_supported(G, sizeof(T) == 8, P.recon, P.rsolve)) return false;
-  FusedGeom g = fused_geom(G, chunk_of(G, zc));
+  FusedGeom g = fused_geom(G, chunk_of(G, zc, sizeof(T) == 8));
   unsigned nb = (unsigned)((int64_t)g.ntx * g.nty * g.nchunks);
   dim3 blk(FTHREADS), grd(nb);
   const bool narrow = sizeof(T) == 4 && narrow_fields<T>(G.nc);
@@ -1159,7 +1182,7 @@ bool launch_step_fused_surr(Fields<const float> U, Fields<float> O, const Grid& 
                             double* red, double* dsmax, const unsigned char* simg, float thr,
                             unsigned long long* nsmooth, hipStream_t st) {
   if (!surrogate_grid(G) || P.rsolve != RS_HLLD) return false;
-  FusedGeom g = fused_geom(G, pick_zc(G));
+  FusedGeom g = fused_geom(G, pick_zc(G, 2));
   unsigned nb = (unsigned)((int64_t)g.ntx * g.nty * g.nchunks);
   dim3 blk(FTHREADS), grd(nb);
 #define PMF_FUSED_S(R) launch_fused_variant<float, R, RS_HLLD, true>(grd, st, U, O, g, P, red, simg, thr, nsmooth)
@@ -1363,9 +1386,7 @@ __device__ __forceinline__ void step_fused_ct_body(const Fields<const T>& U, con
                                                    const FusedGeom& g, const StepParams<T>& P,
                                                    const SrcParams<T>& src = SrcParams<T>{}) {
   __shared__ FusedLds<T, SRC, dxy_in_lds<RECON, false>(), EDGES> lds;
-  const int nwg = gridDim.x;
-  int w = blockIdx.x;
-  if ((nwg & 7) == 0) w = (w & 7) * (nwg >> 3) + (w >> 3);
+  const int w = xcd_tile();
   unsigned none = 0;
   (void)fused_item<T, RECON, RS, false, SRC, NARROW, true, false, EDGES>(U, O, g, P, w, lds, nullptr, nullptr, 0.f,
                                                                          none, src, nullptr, ctp);
@@ -1415,7 +1436,7 @@ bool launch_step_fused_ct(Fields<const T> U, Fields<T> O, T* ctp, const Grid& G,
                           hipStream_t st, int zc, const SrcParams<T>* src, bool want_edges, bool* edges) {
   if (edges) *edges = false;
   if (!fused_supported(G, sizeof(T) == 8, P.recon, P.rsolve) || !all_periodic(G)) return false;
-  FusedGeom g = fused_geom(G, chunk_of(G, zc));
+  FusedGeom g = fused_geom(G, chunk_of(G, zc, sizeof(T) == 8));
   dim3 blk(FTHREADS), grd((unsigned)((int64_t)g.ntx * g.nty * g.nchunks));
   const bool narrow = sizeof(T) == 4 && narrow_fields<T>(G.nc);
 #define PMF_CT(R, S)                                                                   \

@@ -5,7 +5,8 @@
 
 namespace pmf {
 
-// boundary.jl:17-31 (0-based): in-range source index and flip sign for one axis.
+// boundary.jl:17-31 (0-based): in-range source index and flip sign for one axis. On a
+// reflecting axis of one cell the second ghost layer's mirror lies outside and is clamped.
 __device__ __forceinline__ int bc_map(int i, int n, int code, float& flip) {
   flip = 1.0f;
   if (code == BC_PERIODIC) {
@@ -15,11 +16,11 @@ __device__ __forceinline__ int bc_map(int i, int n, int code, float& flip) {
   if (code == BC_OUTFLOW) return i < 0 ? 0 : (i >= n ? n - 1 : i);
   if (i < 0) {
     flip = -1.0f;
-    return -1 - i;
+    return min(-1 - i, n - 1);
   }
   if (i >= n) {
     flip = -1.0f;
-    return 2 * n - 1 - i;
+    return max(2 * n - 1 - i, 0);
   }
   return i;
 }

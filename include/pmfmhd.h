@@ -156,11 +156,11 @@ int pmf_set_chunk(pmf_state* s, int32_t zc);
  * step. Small grids whose built-in choice is shorter than 4 planes keep that one if it is
  * faster; the depth returned is then the fastest of 4..128. */
 int pmf_autotune(pmf_state* s, int32_t reps, int32_t* zc_out, double* ms_out);
-/* Kernel of the CT (:ref) step. By default a constrained-transport state steps (plain,
- * drag and radiation steps alike) on the fused z-marching kernel, which solves every face
- * once with the :ref algorithm (integrator_ref.jl:83-139, 222-258); per_cell != 0
- * selects the per-cell kernel of integrator_ref.jl:189-220 instead. No counterpart in the
- * reference (one kernel there); results agree to rounding. */
+/* Kernel of the :ref step. By default a state's :ref steps (constrained transport and
+ * GLM; plain, drag and radiation steps alike) run on the fused z-marching kernel, which
+ * solves every face once with the :ref algorithm (integrator_ref.jl:83-139, 222-258);
+ * per_cell != 0 selects the per-cell kernel of integrator_ref.jl:189-220 instead. No
+ * counterpart in the reference (one kernel there); results agree to rounding. */
 int pmf_set_ct_kernel(pmf_state* s, int32_t per_cell);
 /* Workspace slots of the fused CT step. The reference's step writes every face's mass and
  * transverse-field fluxes and every cell's EMF to slots 3-14 of the CTState buffer, and

@@ -42,10 +42,24 @@ double smax_device(pmf_state* s) {
   return s->hval[0];
 }
 
+// Whether the :ref integrator's GLM steps run on the fused kernel: the same scheme (PLM the
+// same bits, PPM to rounding) with every face solved and every cell predicted once. It was
+// the faster one on every grid measured: 8^3 34 -> 13.5 us, 32^3 35 -> 14, 128^3 577 -> 110,
+// 200x125x83 MonCen with boundaries 519 -> 113 (float); 160^3 float64 2731 -> 572; 128^3 drag
+// and radiation steps 461-1095 -> 162-231 (float), 1176-1598 -> 451-562 (float64). The per-cell
+// kernel keeps reflecting axes of one cell, grids whose partial maxima do
+// not fit the workspace, and pmf_set_ct_kernel.
+bool ref_on_fused(const pmf_state* s) {
+  const bool f64 = s->p.precision == PMF_F64;
+  return !s->percell && s->p.solver == PMF_SOLVER_GLM &&
+         fused_supported(s->G, s->p.precision, s->p.recon, s->p.riemann) && fused_blocks(s->G, f64, s->zc) <= s->nred;
+}
+
 // One step from fields `in` into fields `out` (integrator_ref.jl:69-172 / the cube launch),
-// then ct_update! on `out` for CT states (ct.jl:158-173). No swap.
+// then ct_update! on `out` for CT states (ct.jl:158-173). No swap. Returns whether the new
+// state's CFL speed is in dval[0].
 template <class T>
-void step_fields(pmf_state* s, Fields<const T> in, Fields<T> out, T* ctp, double dt, double ch, double decay,
+bool step_fields(pmf_state* s, Fields<const T> in, Fields<T> out, T* ctp, double dt, double ch, double decay,
                  int integrator) {
   const bool ct = s->p.solver == PMF_SOLVER_CT;
   bool edges = false;  // CT: the step kernel formed the edge EMFs
@@ -56,7 +70,8 @@ void step_fields(pmf_state* s, Fields<const T> in, Fields<T> out, T* ctp, double
                 "integrators)");
   if (!ct && !(ch > 0.0)) throw Error("step! needs the GLM cleaning speed `ch` (GLM states)");
   if (ct && !ctp) throw Error("ct_update! needs a CT state");
-  if (integrator == PMF_INTEGRATOR_CUBE) {
+  const bool fused = integrator == PMF_INTEGRATOR_CUBE || ref_on_fused(s);
+  if (fused) {
     if (!fused_supported(s->G, s->p.precision, s->p.recon, s->p.riemann))
       throw Error("step_cube!: the fused kernel needs every axis at least one cell and reflecting axes two "
                   "(got " + std::to_string(s->p.nx) + "x" + std::to_string(s->p.ny) + "x" + std::to_string(s->p.nz) +
@@ -66,7 +81,7 @@ void step_fields(pmf_state* s, Fields<const T> in, Fields<T> out, T* ctp, double
         launch_step_fused<T>(in, out, s->G, make_params<T>(s, dt, ch, decay), s->red, s->dval, s->st, s->zc);
     mark(s);
     if (!done) throw Error("step_cube!: fused kernel unavailable for this configuration");
-  } else if (ct && !s->ct_percell && fused_supported(s->G, s->p.precision, s->p.recon, s->p.riemann) &&
+  } else if (ct && !s->percell && fused_supported(s->G, s->p.precision, s->p.recon, s->p.riemann) &&
              all_periodic(s->G)) {
     // the same :ref algorithm with each face solved once (z-marching tiles); where the
     // variant allows, the edge EMFs of ct_update! come out of the same kernel
@@ -86,6 +101,7 @@ void step_fields(pmf_state* s, Fields<const T> in, Fields<T> out, T* ctp, double
     launch_ct_update<T>(out, ctp, s->G, T(dt) / T(s->p.dx), false, s->st, &Pw, s->red, s->dval, edges);
     hip_check(hipGetLastError(), "ct_update launch");
   }
+  return fused || ct;
 }
 
 // The drag / radiation-coupled steps (step_ref_drag!, step_ref_radiation!,
@@ -118,7 +134,7 @@ template <class T> void drag_work(T q, T& A, T& C, T& D) {
 }
 
 template <class T>
-void step_fields_src(pmf_state* s, Fields<const T> in, Fields<T> out, T* ctp, double dt, double ch, double decay,
+bool step_fields_src(pmf_state* s, Fields<const T> in, Fields<T> out, T* ctp, double dt, double ch, double decay,
                      int integrator, const SourceCall& a) {
   const bool ct = s->p.solver == PMF_SOLVER_CT;
   const bool cube = integrator == PMF_INTEGRATOR_CUBE;
@@ -174,7 +190,8 @@ void step_fields_src(pmf_state* s, Fields<const T> in, Fields<T> out, T* ctp, do
   } else if (a.flags & PMF_SRC_GLOBAL_FALLBACK) {
     P.rsolve = RS_LLF;
   }
-  if (cube) {
+  const bool fused = cube || ref_on_fused(s);
+  if (fused) {
     if (!fused_supported(s->G, s->p.precision, P.recon, P.rsolve))
       throw Error(std::string(what) + ": the fused kernel needs every axis at least one cell and reflecting axes two "
                                       "(got " + std::to_string(s->p.nx) + "x" + std::to_string(s->p.ny) + "x" +
@@ -183,7 +200,7 @@ void step_fields_src(pmf_state* s, Fields<const T> in, Fields<T> out, T* ctp, do
     bool done = launch_step_fused<T>(in, out, s->G, P, s->red, s->dval, s->st, s->zc, &S);
     mark(s);
     if (!done) throw Error(std::string(what) + ": fused kernel unavailable for this configuration");
-  } else if (ct && !s->ct_percell && S.check != CHECK_MASKED && S.check != CHECK_GLOBAL &&
+  } else if (ct && !s->percell && S.check != CHECK_MASKED && S.check != CHECK_GLOBAL &&
              fused_supported(s->G, s->p.precision, P.recon, P.rsolve) && all_periodic(s->G)) {
     // the CT :ref step with sources, each face solved once
     mark(s);
@@ -202,26 +219,28 @@ void step_fields_src(pmf_state* s, Fields<const T> in, Fields<T> out, T* ctp, do
                         &Pw, s->red, s->dval);
     hip_check(hipGetLastError(), "ct_update launch");
   }
+  return fused || ct;
 }
 
 void do_step_src(pmf_state* s, double dt, double ch, double decay, int integrator, const SourceCall& a) {
   check_fields(s);
+  bool folded;
   if (s->p.precision == PMF_F64)
-    step_fields_src<double>(s, cfields_at<double>(s->U, s->nc), fields_at<double>(s->S, s->nc), (double*)s->ct, dt,
+    folded = step_fields_src<double>(s, cfields_at<double>(s->U, s->nc), fields_at<double>(s->S, s->nc), (double*)s->ct, dt,
                             ch, decay, integrator, a);
   else
-    step_fields_src<float>(s, cfields_at<float>(s->U, s->nc), fields_at<float>(s->S, s->nc), (float*)s->ct, dt, ch,
-                           decay, integrator, a);
+    folded = step_fields_src<float>(s, cfields_at<float>(s->U, s->nc), fields_at<float>(s->S, s->nc), (float*)s->ct,
+                                    dt, ch, decay, integrator, a);
   std::swap(s->U, s->S);
-  // the fused GLM epilogue or the CT cell-field pass reduced the new state's CFL speed
-  s->smax_valid = (integrator == PMF_INTEGRATOR_CUBE && s->p.solver == PMF_SOLVER_GLM) || s->p.solver == PMF_SOLVER_CT;
+  s->smax_valid = folded;
 }
 
 // step_ref! / step_cube! on the state's own fields: into scratch, then swap.
 void do_step(pmf_state* s, double dt, double ch, double decay, int integrator) {
   check_fields(s);
+  bool folded;  // by the fused GLM epilogue or the CT cell-field pass
   if (s->p.precision == PMF_F64)
-    step_fields<double>(s, cfields_at<double>(s->U, s->nc), fields_at<double>(s->S, s->nc), (double*)s->ct, dt, ch,
+    folded = step_fields<double>(s, cfields_at<double>(s->U, s->nc), fields_at<double>(s->S, s->nc), (double*)s->ct, dt, ch,
                         decay, integrator);
   else
     step_fields<float>(s, cfields_at<float>(s->U, s->nc), fields_at<float>(s->S, s->nc), (float*)s->ct, dt, ch,
@@ -299,6 +318,7 @@ void create_state(const pmf_params* pp, pmf_state** out, bool with_fields) {
     const size_t nred = std::max<size_t>(size_t(kRedBlocks) * kRedSlots,
                                          size_t(std::max(fused_blocks(s->G, f64), fused_blocks(s->G, f64, kMinChunk))));
     hip_check(hipMalloc(&s->red, sizeof(double) * nred), "hipMalloc(red)");
+    s->nred = int64_t(nred);
     hip_check(hipMalloc(&s->dval, sizeof(double) * 64), "hipMalloc(dval)");
     hip_check(hipHostMalloc((void**)&s->hval, sizeof(double) * 64, hipHostMallocDefault), "hipHostMalloc");
     sync(s);
@@ -436,7 +456,7 @@ int pmf_compute_dt(pmf_state* s, double cfl, double* dt, double* smax) {
 int pmf_set_ct_kernel(pmf_state* s, int32_t per_cell) {
   return guard([&] {
     check_state(s);
-    s->ct_percell = per_cell != 0;
+    s->percell = per_cell != 0;
   });
 }
 
@@ -895,15 +915,17 @@ int pmf_step_into_static(const pmf_params* p, const void* const* U, void* const*
     s.esz = p->precision == PMF_F64 ? 8 : 4;
     s.st = (hipStream_t)hip_stream;
     s.red = w;
+    s.nred = kStaticPartials;
     s.dval = w + kStaticPartials;
-    const bool folded = p->solver == PMF_SOLVER_CT || integrator == PMF_INTEGRATOR_CUBE;
     if (p->precision == PMF_F64) {
-      step_fields<double>(&s, cfields_from<double>(U), fields_from<double>(O), (double*)ct, dt, ch, decay, integrator);
+      const bool folded =
+          step_fields<double>(&s, cfields_from<double>(U), fields_from<double>(O), (double*)ct, dt, ch, decay, integrator);
       if (smax_dev && !folded)
         launch_wavespeed<double>(cfields_from<double>((const void* const*)O), s.G, make_params<double>(&s, 0, 0, 1),
                                  s.red, s.dval, s.st);
     } else {
-      step_fields<float>(&s, cfields_from<float>(U), fields_from<float>(O), (float*)ct, dt, ch, decay, integrator);
+      const bool folded =
+          step_fields<float>(&s, cfields_from<float>(U), fields_from<float>(O), (float*)ct, dt, ch, decay, integrator);
       if (smax_dev && !folded)
         launch_wavespeed<float>(cfields_from<float>((const void* const*)O), s.G, make_params<float>(&s, 0, 0, 1),
                                 s.red, s.dval, s.st);

@@ -46,6 +46,7 @@ struct pmf_state {
   void* S = nullptr;     // 9*nc scratch
   void* ct = nullptr;    // 21*nc (CT only)
   double* red = nullptr; // reduction partials
+  int64_t nred = 0;      // doubles in red
   double* dval = nullptr;  // device scalars: [0]=smax [1..3]=divb [4..11]=totals [12]=face div
   double* hval = nullptr;  // pinned host mirror of dval
   hipStream_t own = nullptr;
@@ -53,7 +54,7 @@ struct pmf_state {
   int device = 0;
   bool smax_valid = false;  // dval[0] holds the CFL speed of the current U
   int zc = 0;               // planes per z chunk of the fused kernel (0 = built-in choice)
-  bool ct_percell = false;  // CT steps on the per-cell kernel even where the fused one applies
+  bool percell = false;  // :ref steps on the per-cell kernel even where the fused one applies
   // CT steps on the fused kernel also write workspace slots 3-14 (face mass and field fluxes,
   // cell EMFs) and form the edge EMFs in a separate pass, as the reference's step does;
   // otherwise the fused kernel forms the edge EMFs itself and leaves slots 3-14 alone

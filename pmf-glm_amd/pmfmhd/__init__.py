@@ -378,8 +378,8 @@ def set_chunk(s: MHDState, zc: int):
 
 
 def set_ct_kernel(s: MHDState, per_cell: bool):
-    """CT steps on the per-cell kernel (True) or, where the grid allows (nx a multiple
-    of 16), on the fused kernel that solves every face once (False, the default)."""
+    """:ref steps (CT and GLM) on the per-cell kernel (True) or on the fused kernel that
+    solves every face once (False, the default)."""
     check(lib().pmf_set_ct_kernel(s.handle, 1 if per_cell else 0))
 
 

@@ -27,18 +27,20 @@ void pmf::set_error(const std::string& msg) { g_err = msg; }
 
 namespace {
 
+// The kernels that fold the CFL speed of a state's fields write it to dval[0] and to the pinned
+// hval[0], so reading it takes one wait and no copy (32^3 host-driven step 25.6 -> 23.8 us).
 double smax_device(pmf_state* s) {
   if (!s->smax_valid) {
     if (s->p.precision == PMF_F64)
       launch_wavespeed<double>(cfields_at<double>(s->U, s->nc), s->G, make_params<double>(s, 0, 0, 1), s->red,
-                               s->dval, s->st);
+                               s->dval, s->st, s->hval);
     else
       launch_wavespeed<float>(cfields_at<float>(s->U, s->nc), s->G, make_params<float>(s, 0, 0, 1), s->red, s->dval,
-                              s->st);
+                              s->st, s->hval);
     hip_check(hipGetLastError(), "wavespeed launch");
     s->smax_valid = true;
   }
-  fetch(s, 0, 1);
+  sync(s);
   return s->hval[0];
 }
 
@@ -57,10 +59,12 @@ bool ref_on_fused(const pmf_state* s) {
 
 // One step from fields `in` into fields `out` (integrator_ref.jl:69-172 / the cube launch),
 // then ct_update! on `out` for CT states (ct.jl:158-173). No swap. Returns whether the new
-// state's CFL speed is in dval[0].
+// state's CFL speed was folded into dval[0] and hval[0]; with fold = false (the caller's
+// arrays, whose speed the state does not keep) that reduction is left out.
 template <class T>
 bool step_fields(pmf_state* s, Fields<const T> in, Fields<T> out, T* ctp, double dt, double ch, double decay,
-                 int integrator) {
+                 int integrator, bool fold) {
+  double* const dsmax = fold ? s->dval : nullptr;
   const bool ct = s->p.solver == PMF_SOLVER_CT;
   bool edges = false;  // CT: the step kernel formed the edge EMFs
   if (integrator != PMF_INTEGRATOR_REF && integrator != PMF_INTEGRATOR_CUBE)
@@ -78,7 +82,8 @@ bool step_fields(pmf_state* s, Fields<const T> in, Fields<T> out, T* ctp, double
                   ")");
     mark(s);
     bool done =
-        launch_step_fused<T>(in, out, s->G, make_params<T>(s, dt, ch, decay), s->red, s->dval, s->st, s->zc);
+        launch_step_fused<T>(in, out, s->G, make_params<T>(s, dt, ch, decay), s->red, dsmax, s->st, s->zc, nullptr,
+                             nullptr, s->hval);
     mark(s);
     if (!done) throw Error("step_cube!: fused kernel unavailable for this configuration");
   } else if (ct && !s->percell && fused_supported(s->G, s->p.precision, s->p.recon, s->p.riemann) &&
@@ -98,10 +103,10 @@ bool step_fields(pmf_state* s, Fields<const T> in, Fields<T> out, T* ctp, double
   if (ct) {
     // ct_update! with the new state's CFL speed folded into dval[0] by its last pass
     const StepParams<T> Pw = make_params<T>(s, 0, 0, 1);
-    launch_ct_update<T>(out, ctp, s->G, T(dt) / T(s->p.dx), false, s->st, &Pw, s->red, s->dval, edges);
+    launch_ct_update<T>(out, ctp, s->G, T(dt) / T(s->p.dx), false, s->st, &Pw, s->red, dsmax, edges, s->hval);
     hip_check(hipGetLastError(), "ct_update launch");
   }
-  return fused || ct;
+  return fold && (fused || ct);
 }
 
 // The drag / radiation-coupled steps (step_ref_drag!, step_ref_radiation!,
@@ -135,7 +140,8 @@ template <class T> void drag_work(T q, T& A, T& C, T& D) {
 
 template <class T>
 bool step_fields_src(pmf_state* s, Fields<const T> in, Fields<T> out, T* ctp, double dt, double ch, double decay,
-                     int integrator, const SourceCall& a) {
+                     int integrator, const SourceCall& a, bool fold) {
+  double* const dsmax = fold ? s->dval : nullptr;
   const bool ct = s->p.solver == PMF_SOLVER_CT;
   const bool cube = integrator == PMF_INTEGRATOR_CUBE;
   const char* what = a.radiation ? (cube ? "step_cube_radiation!" : "step_ref_radiation!")
@@ -197,7 +203,7 @@ bool step_fields_src(pmf_state* s, Fields<const T> in, Fields<T> out, T* ctp, do
                                       "(got " + std::to_string(s->p.nx) + "x" + std::to_string(s->p.ny) + "x" +
                   std::to_string(s->p.nz) + ")");
     mark(s);
-    bool done = launch_step_fused<T>(in, out, s->G, P, s->red, s->dval, s->st, s->zc, &S);
+    bool done = launch_step_fused<T>(in, out, s->G, P, s->red, dsmax, s->st, s->zc, &S, nullptr, s->hval);
     mark(s);
     if (!done) throw Error(std::string(what) + ": fused kernel unavailable for this configuration");
   } else if (ct && !s->percell && S.check != CHECK_MASKED && S.check != CHECK_GLOBAL &&
@@ -216,10 +222,10 @@ bool step_fields_src(pmf_state* s, Fields<const T> in, Fields<T> out, T* ctp, do
     // compensated faces exactly when GLM would compensate cell B (integrator_ref.jl:255-256)
     const StepParams<T> Pw = make_params<T>(s, 0, 0, 1);
     launch_ct_update<T>(out, ctp, s->G, T(dt) / T(s->p.dx), a.radiation && (a.flags & PMF_SRC_TRACK_MAGNETIC), s->st,
-                        &Pw, s->red, s->dval);
+                        &Pw, s->red, dsmax, false, s->hval);
     hip_check(hipGetLastError(), "ct_update launch");
   }
-  return fused || ct;
+  return fold && (fused || ct);
 }
 
 void do_step_src(pmf_state* s, double dt, double ch, double decay, int integrator, const SourceCall& a) {
@@ -227,10 +233,10 @@ void do_step_src(pmf_state* s, double dt, double ch, double decay, int integrato
   bool folded;
   if (s->p.precision == PMF_F64)
     folded = step_fields_src<double>(s, cfields_at<double>(s->U, s->nc), fields_at<double>(s->S, s->nc), (double*)s->ct, dt,
-                            ch, decay, integrator, a);
+                            ch, decay, integrator, a, true);
   else
     folded = step_fields_src<float>(s, cfields_at<float>(s->U, s->nc), fields_at<float>(s->S, s->nc), (float*)s->ct,
-                                    dt, ch, decay, integrator, a);
+                                    dt, ch, decay, integrator, a, true);
   std::swap(s->U, s->S);
   s->smax_valid = folded;
 }
@@ -240,15 +246,13 @@ void do_step(pmf_state* s, double dt, double ch, double decay, int integrator) {
   check_fields(s);
   bool folded;  // by the fused GLM epilogue or the CT cell-field pass
   if (s->p.precision == PMF_F64)
-    folded = step_fields<double>(s, cfields_at<double>(s->U, s->nc), fields_at<double>(s->S, s->nc), (double*)s->ct, dt, ch,
-                        decay, integrator);
+    folded = step_fields<double>(s, cfields_at<double>(s->U, s->nc), fields_at<double>(s->S, s->nc), (double*)s->ct, dt,
+                                 ch, decay, integrator, true);
   else
-    step_fields<float>(s, cfields_at<float>(s->U, s->nc), fields_at<float>(s->S, s->nc), (float*)s->ct, dt, ch,
-                       decay, integrator);
+    folded = step_fields<float>(s, cfields_at<float>(s->U, s->nc), fields_at<float>(s->S, s->nc), (float*)s->ct, dt, ch,
+                                decay, integrator, true);
   std::swap(s->U, s->S);
-  // the fused GLM epilogue or the CT cell-field pass reduced the new state's CFL speed
-  // into dval[0]
-  s->smax_valid = (integrator == PMF_INTEGRATOR_CUBE && s->p.solver == PMF_SOLVER_GLM) || s->p.solver == PMF_SOLVER_CT;
+  s->smax_valid = folded;
 }
 
 }  // namespace
@@ -539,17 +543,22 @@ void advance_steps(pmf_state* s, int64_t nsteps, double cfl, double fac, double 
     launch_wavespeed<T>(cfields_at<T>(s->U, s->nc), s->G, base, s->red, s->dval, s->st);
     hip_check(hipGetLastError(), "wavespeed launch");
   }
+  // each step leaves its partial speeds in red; the next step's scalars fold them themselves
+  const int64_t nb = fused_blocks(s->G, sizeof(T) == 8, s->zc);
   for (int64_t k = 0; k < nsteps; ++k) {
-    launch_step_params<T>(s->dval, base, Pd, clock, cfl, fac, cr, s->p.dx, k == 0, s->st);
+    launch_step_params<T>(s->dval, s->red, k == 0 ? 0 : nb, base, Pd, clock, cfl, fac, cr, s->p.dx, k == 0, s->st);
     mark(s);
     const bool done = launch_step_fused<T>(cfields_at<T>(s->U, s->nc), fields_at<T>(s->S, s->nc), s->G, base, s->red,
-                                           s->dval, s->st, s->zc, nullptr, Pd);
+                                           nullptr, s->st, s->zc, nullptr, Pd);
     mark(s);
     if (!done) throw Error("pmf_advance: fused kernel unavailable for this configuration");
     hip_check(hipGetLastError(), "step launch");
     std::swap(s->U, s->S);
+    s->smax_valid = false;
   }
-  s->smax_valid = true;  // the last step folded its new state's speed into dval[0]
+  launch_fold_max(s->red, nb, s->dval, s->hval, s->st);
+  hip_check(hipGetLastError(), "fold launch");
+  s->smax_valid = true;
 }
 }  // namespace
 }  // extern "C++"
@@ -627,10 +636,10 @@ int pmf_autotune(pmf_state* s, int32_t reps, int32_t* zc_out, double* ms_out) {
                                         nullptr, !s->ct_fill_workspace);
           else if (s->p.precision == PMF_F64)
             step_fields<double>(s, cfields_at<double>(s->U, s->nc), fields_at<double>(s->S, s->nc), nullptr, dt, ch,
-                                1.0, PMF_INTEGRATOR_CUBE);
+                                1.0, PMF_INTEGRATOR_CUBE, true);
           else
             step_fields<float>(s, cfields_at<float>(s->U, s->nc), fields_at<float>(s->S, s->nc), nullptr, dt, ch, 1.0,
-                               PMF_INTEGRATOR_CUBE);
+                               PMF_INTEGRATOR_CUBE, true);
           hip_check(hipGetLastError(), "autotune launch");
         };
         launch();  // warm-up
@@ -821,11 +830,13 @@ int pmf_step_into(pmf_state* s, const void* const* U, void* const* O, void* ct, 
   return guard([&] {
     check_state(s);
     if (!U || !O) throw Error("null field array");
-    s->smax_valid = false;  // dval[0] now describes the caller's output arrays
+    s->smax_valid = false;
     if (s->p.precision == PMF_F64)
-      step_fields<double>(s, cfields_from<double>(U), fields_from<double>(O), (double*)ct, dt, ch, decay, integrator);
+      step_fields<double>(s, cfields_from<double>(U), fields_from<double>(O), (double*)ct, dt, ch, decay, integrator,
+                          false);
     else
-      step_fields<float>(s, cfields_from<float>(U), fields_from<float>(O), (float*)ct, dt, ch, decay, integrator);
+      step_fields<float>(s, cfields_from<float>(U), fields_from<float>(O), (float*)ct, dt, ch, decay, integrator,
+                         false);
   });
 }
 
@@ -919,13 +930,15 @@ int pmf_step_into_static(const pmf_params* p, const void* const* U, void* const*
     s.dval = w + kStaticPartials;
     if (p->precision == PMF_F64) {
       const bool folded =
-          step_fields<double>(&s, cfields_from<double>(U), fields_from<double>(O), (double*)ct, dt, ch, decay, integrator);
+          step_fields<double>(&s, cfields_from<double>(U), fields_from<double>(O), (double*)ct, dt, ch, decay,
+                              integrator, smax_dev != nullptr);
       if (smax_dev && !folded)
         launch_wavespeed<double>(cfields_from<double>((const void* const*)O), s.G, make_params<double>(&s, 0, 0, 1),
                                  s.red, s.dval, s.st);
     } else {
       const bool folded =
-          step_fields<float>(&s, cfields_from<float>(U), fields_from<float>(O), (float*)ct, dt, ch, decay, integrator);
+          step_fields<float>(&s, cfields_from<float>(U), fields_from<float>(O), (float*)ct, dt, ch, decay, integrator,
+                             smax_dev != nullptr);
       if (smax_dev && !folded)
         launch_wavespeed<float>(cfields_from<float>((const void* const*)O), s.G, make_params<float>(&s, 0, 0, 1),
                                 s.red, s.dval, s.st);
@@ -968,7 +981,7 @@ int pmf_step_sources_into(pmf_state* s, const void* const* U, void* const* O, vo
   return guard([&] {
     check_state(s);
     if (!U || !O) throw Error("null field array");
-    s->smax_valid = false;  // the fused epilogue leaves dval[0] describing the caller's output arrays
+    s->smax_valid = false;
     SourceCall a;
     a.radiation = correction != nullptr;
     a.impulse = drag_impulse;
@@ -978,10 +991,10 @@ int pmf_step_sources_into(pmf_state* s, const void* const* U, void* const* O, vo
       for (int d = 0; d < 3; ++d) a.v0[d] = target_velocity[d];
     if (s->p.precision == PMF_F64)
       step_fields_src<double>(s, cfields_from<double>(U), fields_from<double>(O), (double*)ct, dt, ch, decay,
-                              integrator, a);
+                              integrator, a, false);
     else
-      step_fields_src<float>(s, cfields_from<float>(U), fields_from<float>(O), (float*)ct, dt, ch, decay, integrator,
-                             a);
+      step_fields_src<float>(s, cfields_from<float>(U), fields_from<float>(O), (float*)ct, dt, ch, decay, integrator, a,
+                             false);
   });
 }
 

@@ -18,8 +18,9 @@ void launch_step_ref(Fields<const T> U, Fields<T> O, T* ctp, const Grid& G, cons
                      hipStream_t st, const SrcParams<T>* S = nullptr);
 
 // Fused tiled step (periodic GLM). Writes per-block CFL maxima of the new state into
-// red (one double per block) and the final max into dsmax. Returns false when the grid
-// shape is not supported by the fused kernel.
+// red (one double per block) and, unless dsmax is null, the final max into *dsmax and, if
+// given, *hsmax (pinned host memory). Returns false when the grid shape is not supported by
+// the fused kernel.
 // zc: planes per z chunk (0 = the built-in choice); src: drag / radiation source terms
 // (nullptr for the plain step).
 // Pd: device-resident step scalars that replace P's (dt, ch, decay) in the kernel (P still
@@ -27,13 +28,17 @@ void launch_step_ref(Fields<const T> U, Fields<T> O, T* ctp, const Grid& G, cons
 template <class T>
 bool launch_step_fused(Fields<const T> U, Fields<T> O, const Grid& G, const StepParams<T>& P, double* red,
                        double* dsmax, hipStream_t st, int zc = 0, const SrcParams<T>* src = nullptr,
-                       const StepParams<T>* Pd = nullptr);
+                       const StepParams<T>* Pd = nullptr, double* hsmax = nullptr);
+// The maximum of red[0 .. nb) into *dsmax and, if given, *hsmax (pinned host memory).
+void launch_fold_max(const double* red, int64_t nb, double* dsmax, double* hsmax, hipStream_t st);
 // The device-side CFL stage of pmf_advance (evolve!'s rule, driver.jl:48-71, evaluated as
-// the host does it): from the speed in dsmax[0], writes the step scalars to Pd and adds
-// the step to clock[0] (reset: sets it), clock[1] = the step's dt.
+// the host does it): from the speed in dsmax[0], or for nb > 0 from the maximum of the
+// previous step's partials red[0 .. nb), writes the step scalars to Pd and adds the step to
+// clock[0] (reset: sets it), clock[1] = the step's dt.
 template <class T>
-void launch_step_params(const double* dsmax, const StepParams<T>& base, StepParams<T>* Pd, double* clock, double cfl,
-                        double glm_ch_fac, double glm_cr, double dx, int reset, hipStream_t st);
+void launch_step_params(const double* dsmax, const double* red, int64_t nb, const StepParams<T>& base,
+                        StepParams<T>* Pd, double* clock, double cfl, double glm_ch_fac, double glm_cr, double dx,
+                        int reset, hipStream_t st);
 bool fused_supported(const Grid& G, int precision, int recon, int rsolve);
 bool all_periodic(const Grid& G);
 bool surrogate_grid(const Grid& G);
@@ -52,7 +57,7 @@ bool launch_step_fused_ct(Fields<const T> U, Fields<T> O, T* ctp, const Grid& G,
 // nsmooth accumulates the number of faces solved by the network.
 bool launch_step_fused_surr(Fields<const float> U, Fields<float> O, const Grid& G, const StepParams<float>& P,
                             double* red, double* dsmax, const unsigned char* simg, float thr,
-                            unsigned long long* nsmooth, hipStream_t st);
+                            unsigned long long* nsmooth, hipStream_t st, double* hsmax);
 // Number of workgroups (one partial maximum each) the fused kernel launches for G in the
 // given precision with z chunks of zc planes (0 = the built-in choice).
 int64_t fused_blocks(const Grid& G, bool f64, int zc = 0);
@@ -102,17 +107,18 @@ void launch_backtrace(T* o1, T* o2, const T* a1, const T* a2, Fields<const T> U,
 
 template <class T>
 void launch_wavespeed(Fields<const T> U, const Grid& G, const StepParams<T>& P, double* red, double* out,
-                      hipStream_t st);
+                      hipStream_t st, double* hout = nullptr);
 template <class T>
 void launch_divb(Fields<const T> U, const Grid& G, T inv2dx, double* red, double* out3, hipStream_t st);
 template <class T> void launch_totals(Fields<const T> U, const Grid& G, double* red, double* out8, hipStream_t st);
 // ct_update! (ct.jl:158-173) on U. With P, red and dsmax: the cell-field pass also folds
-// the CFL speed of the finished state into *dsmax (device), as the fused GLM step does.
+// the CFL speed of the finished state into *dsmax (device) and, if given, *hsmax (pinned host
+// memory), as the fused GLM step does.
 // have_edges: slots 15-17 already hold this step's edge EMFs (formed by the step kernel).
 template <class T>
 void launch_ct_update(Fields<T> U, T* ctp, const Grid& G, T dtdx, bool compensate, hipStream_t st,
                       const StepParams<T>* P = nullptr, double* red = nullptr, double* dsmax = nullptr,
-                      bool have_edges = false);
+                      bool have_edges = false, double* hsmax = nullptr);
 template <class T> void launch_divb_face(const T* ctp, const Grid& G, T invdx, double* red, double* out, hipStream_t st);
 template <class T>
 void launch_ct_install(Fields<T> U, T* ctp, const Grid& G, hipStream_t st);

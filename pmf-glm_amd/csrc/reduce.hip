@@ -76,9 +76,10 @@ static inline unsigned red_grid(int64_t n) {
 }
 
 // Final fold of nb partial slots of (NV sums, NM maxima) laid out as
-// [s0 c0 s1 c1 ... m0 m1 ...] per block.
+// [s0 c0 s1 c1 ... m0 m1 ...] per block; hout (pinned host memory, may be null) gets them too.
 template <int NV, int NM>
-__global__ __launch_bounds__(kBlk) void k_fold_final(const double* __restrict__ red, int nb, double* __restrict__ out) {
+__global__ __launch_bounds__(kBlk) void k_fold_final(const double* __restrict__ red, int nb, double* __restrict__ out,
+                                                     double* __restrict__ hout = nullptr) {
   KSum sums[NV > 0 ? NV : 1];
   double maxs[NM > 0 ? NM : 1];
   for (int v = 0; v < NV; ++v) sums[v] = KSum{0.0, 0.0};
@@ -90,8 +91,14 @@ __global__ __launch_bounds__(kBlk) void k_fold_final(const double* __restrict__ 
   }
   block_fold<NV, NM>(sums, maxs);
   if (threadIdx.x == 0) {
-    for (int v = 0; v < NV; ++v) out[v] = sums[v].s + sums[v].c;
-    for (int m = 0; m < NM; ++m) out[NV + m] = maxs[m];
+    for (int v = 0; v < NV; ++v) {
+      out[v] = sums[v].s + sums[v].c;
+      if (hout) hout[v] = out[v];
+    }
+    for (int m = 0; m < NM; ++m) {
+      out[NV + m] = maxs[m];
+      if (hout) hout[NV + m] = maxs[m];
+    }
   }
 }
 
@@ -126,10 +133,10 @@ __global__ __launch_bounds__(kBlk) void k_wavespeed(Fields<const T> U, Grid G, S
 
 template <class T>
 void launch_wavespeed(Fields<const T> U, const Grid& G, const StepParams<T>& P, double* red, double* out,
-                      hipStream_t st) {
+                      hipStream_t st, double* hout) {
   unsigned nb = red_grid(G.nc);
   hipLaunchKernelGGL((k_wavespeed<T>), dim3(nb), dim3(kBlk), 0, st, U, G, P, red);
-  hipLaunchKernelGGL((k_fold_final<0, 1>), dim3(1), dim3(kBlk), 0, st, red, (int)nb, out);
+  hipLaunchKernelGGL((k_fold_final<0, 1>), dim3(1), dim3(kBlk), 0, st, red, (int)nb, out, hout);
 }
 
 // ---- centred div B (diagnostics.jl:6-21): max and float64 sum of squares --------
@@ -175,7 +182,7 @@ template <class T>
 void launch_divb(Fields<const T> U, const Grid& G, T inv2dx, double* red, double* out, hipStream_t st) {
   unsigned nb = red_grid(G.nc);
   hipLaunchKernelGGL((k_divb<T>), dim3(nb), dim3(kBlk), 0, st, U, G, inv2dx, red);
-  hipLaunchKernelGGL((k_fold_final<1, 1>), dim3(1), dim3(kBlk), 0, st, red, (int)nb, out);
+  hipLaunchKernelGGL((k_fold_final<1, 1>), dim3(1), dim3(kBlk), 0, st, red, (int)nb, out, nullptr);
 }
 
 // ---- conserved totals (diagnostics.jl:44-55) -------------------------------------
@@ -197,7 +204,7 @@ __global__ __launch_bounds__(kBlk) void k_totals(Fields<const T> U, Grid G, doub
 template <class T> void launch_totals(Fields<const T> U, const Grid& G, double* red, double* out8, hipStream_t st) {
   unsigned nb = red_grid(G.nc);
   hipLaunchKernelGGL((k_totals<T>), dim3(nb), dim3(kBlk), 0, st, U, G, red);
-  hipLaunchKernelGGL((k_fold_final<8, 0>), dim3(1), dim3(kBlk), 0, st, red, (int)nb, out8);
+  hipLaunchKernelGGL((k_fold_final<8, 0>), dim3(1), dim3(kBlk), 0, st, red, (int)nb, out8, nullptr);
 }
 
 // ---- constrained transport (ct.jl) -----------------------------------------------
@@ -300,7 +307,7 @@ __global__ __launch_bounds__(kBlk) void k_ct_bcc_cfl(Fields<T> U, const T* __res
 
 template <class T>
 void launch_ct_update(Fields<T> U, T* ctp, const Grid& G, T dtdx, bool compensate, hipStream_t st,
-                      const StepParams<T>* P, double* red, double* dsmax, bool have_edges) {
+                      const StepParams<T>* P, double* red, double* dsmax, bool have_edges, double* hsmax) {
   dim3 blk(kBlk), grd((unsigned)((G.nc + kBlk - 1) / kBlk));
   if (!have_edges) hipLaunchKernelGGL((k_ct_emf<T>), grd, blk, 0, st, ctp, G);
   if (compensate) hipLaunchKernelGGL((k_ct_faces<T, true>), grd, blk, 0, st, ctp, G, dtdx);
@@ -308,7 +315,7 @@ void launch_ct_update(Fields<T> U, T* ctp, const Grid& G, T dtdx, bool compensat
   if (P && red && dsmax) {
     const unsigned nb = red_grid(G.nc);
     hipLaunchKernelGGL((k_ct_bcc_cfl<T>), dim3(nb), blk, 0, st, U, ctp, G, *P, red);
-    hipLaunchKernelGGL((k_fold_final<0, 1>), dim3(1), blk, 0, st, red, (int)nb, dsmax);
+    hipLaunchKernelGGL((k_fold_final<0, 1>), dim3(1), blk, 0, st, red, (int)nb, dsmax, hsmax);
   } else {
     hipLaunchKernelGGL((k_ct_bcc<T>), grd, blk, 0, st, U, ctp, G);
   }
@@ -334,7 +341,7 @@ __global__ __launch_bounds__(kBlk) void k_divb_face(const T* __restrict__ ctp, G
 template <class T> void launch_divb_face(const T* ctp, const Grid& G, T invdx, double* red, double* out, hipStream_t st) {
   unsigned nb = red_grid(G.nc);
   hipLaunchKernelGGL((k_divb_face<T>), dim3(nb), dim3(kBlk), 0, st, ctp, G, invdx, red);
-  hipLaunchKernelGGL((k_fold_final<0, 1>), dim3(1), dim3(kBlk), 0, st, red, (int)nb, out);
+  hipLaunchKernelGGL((k_fold_final<0, 1>), dim3(1), dim3(kBlk), 0, st, red, (int)nb, out, nullptr);
 }
 
 // ct.jl:205-219: cell B <- face average, E keeps the thermal pressure, psi <- 0.
@@ -389,11 +396,11 @@ void launch_ct_curl(const T* Ax, const T* Ay, const T* Az, T* bx, T* by, T* bz, 
 
 #define PMF_INST(T)                                                                                             \
   template void launch_wavespeed<T>(Fields<const T>, const Grid&, const StepParams<T>&, double*, double*,       \
-                                    hipStream_t);                                                               \
+                                    hipStream_t, double*);                                                               \
   template void launch_divb<T>(Fields<const T>, const Grid&, T, double*, double*, hipStream_t);                  \
   template void launch_totals<T>(Fields<const T>, const Grid&, double*, double*, hipStream_t);                  \
   template void launch_ct_update<T>(Fields<T>, T*, const Grid&, T, bool, hipStream_t, const StepParams<T>*, double*, \
-                                     double*, bool);                                                               \
+                                     double*, bool, double*);                                                               \
   template void launch_divb_face<T>(const T*, const Grid&, T, double*, double*, hipStream_t);                    \
   template void launch_ct_install<T>(Fields<T>, T*, const Grid&, hipStream_t);                                   \
   template void launch_ct_curl<T>(const T*, const T*, const T*, T*, T*, T*, const Grid&, T, hipStream_t);

@@ -992,28 +992,56 @@ template <class T> inline bool narrow_fields(int64_t nc) {
   return (uint64_t)nc * sizeof(T) < (1ull << 32);
 }
 
-__global__ __launch_bounds__(256) void k_fold_max_flat(const double* __restrict__ red, int nb, double* __restrict__ out) {
-  __shared__ double sh[4];
-  double m = 0.0;
-  for (int b = threadIdx.x; b < nb; b += 256) m = nanmax(m, red[b]);
+// Maximum of red[0 .. nb), NaN if one is; every thread of the one block of 1024 gets it. Eight
+// loads in flight a thread: with 256 threads and one load at a time the 22016 partials of a
+// 512^3 step took 37 us; the 2816 of 256^3, 5.0.
+__device__ __forceinline__ double fold_max(const double* __restrict__ red, int nb, double* sh) {
+  double m[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  for (int b = threadIdx.x; b < nb; b += 8 * 1024) {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) m = nanmax(m, __shfl_xor(m, o, 64));
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = m;
+    for (int k = 0; k < 8; ++k) m[k] = nanmax(m[k], red[min(b + k * 1024, nb - 1)]);
+  }
+#pragma unroll
+  for (int k = 4; k > 0; k >>= 1)
+    for (int j = 0; j < k; ++j) m[j] = nanmax(m[j], m[j + k]);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m[0] = nanmax(m[0], __shfl_xor(m[0], o, 64));
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = m[0];
   __syncthreads();
-  if (threadIdx.x == 0) out[0] = nanmax(nanmax(sh[0], sh[1]), nanmax(sh[2], sh[3]));
+  double r = sh[0];
+#pragma unroll
+  for (int k = 1; k < 16; ++k) r = nanmax(r, sh[k]);
+  return r;
+}
+
+__global__ __launch_bounds__(1024) void k_fold_max_flat(const double* __restrict__ red, int nb, double* __restrict__ out,
+                                                        double* __restrict__ hout) {
+  __shared__ double sh[16];
+  const double r = fold_max(red, nb, sh);
+  if (threadIdx.x == 0) {
+    out[0] = r;
+    if (hout) hout[0] = r;
+  }
+}
+
+void launch_fold_max(const double* red, int64_t nb, double* dsmax, double* hsmax, hipStream_t st) {
+  hipLaunchKernelGGL(k_fold_max_flat, dim3(1), dim3(1024), 0, st, red, (int)nb, dsmax, hsmax);
 }
 
 // The device-side CFL stage of pmf_advance: evolve!'s step rule (driver.jl:48-71) from
 // the speed the previous step folded into dsmax[0], in the same operations and
 // precisions as the host path (pmf_compute_dt, pmf_evolve, decay_of, make_params), so
-// that a step with device-resident scalars is the host-driven step bit for bit.
+// that a step with device-resident scalars is the host-driven step bit for bit. nb > 0: folds
+// that speed from the previous step's partials itself, one launch fewer between steps.
 template <class T>
-__global__ __launch_bounds__(64) void k_step_params(const double* __restrict__ dsmax, StepParams<T> base,
-                                                    StepParams<T>* __restrict__ Pd, double* __restrict__ clock,
-                                                    double cfl, double fac, double cr, double dx, int reset) {
+__global__ __launch_bounds__(1024) void k_step_params(const double* __restrict__ dsmax, const double* __restrict__ red,
+                                                      int nb, StepParams<T> base, StepParams<T>* __restrict__ Pd,
+                                                      double* __restrict__ clock, double cfl, double fac, double cr,
+                                                      double dx, int reset) {
 #pragma clang fp contract(off)
+  __shared__ double sh[16];
+  const double sm = nb > 0 ? fold_max(red, nb, sh) : dsmax[0];
   if (threadIdx.x != 0) return;
-  const double sm = dsmax[0];
   double dtf, ch, decay;
   if constexpr (sizeof(T) == 8) {
     const double dt = cfl * dx / (sm < __DBL_EPSILON__ ? __DBL_EPSILON__ : sm);
@@ -1044,15 +1072,16 @@ __global__ __launch_bounds__(64) void k_step_params(const double* __restrict__ d
 }
 
 template <class T>
-void launch_step_params(const double* dsmax, const StepParams<T>& base, StepParams<T>* Pd, double* clock, double cfl,
-                        double glm_ch_fac, double glm_cr, double dx, int reset, hipStream_t st) {
-  hipLaunchKernelGGL((k_step_params<T>), dim3(1), dim3(64), 0, st, dsmax, base, Pd, clock, cfl, glm_ch_fac, glm_cr, dx,
-                     reset);
+void launch_step_params(const double* dsmax, const double* red, int64_t nb, const StepParams<T>& base,
+                        StepParams<T>* Pd, double* clock, double cfl, double glm_ch_fac, double glm_cr, double dx,
+                        int reset, hipStream_t st) {
+  hipLaunchKernelGGL((k_step_params<T>), dim3(1), dim3(nb > 0 ? 1024 : 64), 0, st, dsmax, red, (int)nb, base, Pd, clock,
+                     cfl, glm_ch_fac, glm_cr, dx, reset);
 }
-template void launch_step_params<float>(const double*, const StepParams<float>&, StepParams<float>*, double*, double,
-                                        double, double, double, int, hipStream_t);
-template void launch_step_params<double>(const double*, const StepParams<double>&, StepParams<double>*, double*,
-                                         double, double, double, double, int, hipStream_t);
+template void launch_step_params<float>(const double*, const double*, int64_t, const StepParams<float>&,
+                                        StepParams<float>*, double*, double, double, double, double, int, hipStream_t);
+template void launch_step_params<double>(const double*, const double*, int64_t, const StepParams<double>&,
+                                         StepParams<double>*, double*, double, double, double, double, int, hipStream_t);
 
 static FusedGeom fused_geom(const Grid& G, int zc) {
   FusedGeom g;
@@ -1146,7 +1175,8 @@ int64_t fused_blocks(const Grid& G, bool f64, int zc) {
 
 template <class T>
 bool launch_step_fused(Fields<const T> U, Fields<T> O, const Grid& G, const StepParams<T>& P, double* red,
-                       double* dsmax, hipStream_t st, int zc, const SrcParams<T>* src, const StepParams<T>* Pd) {
+                       double* dsmax, hipStream_t st, int zc, const SrcParams<T>* src, const StepParams<T>* Pd,
+                       double* hsmax) {
   if (!fused_supported(G, sizeof(T) == 8, P.recon, P.rsolve)) return false;
   FusedGeom g = fused_geom(G, chunk_of(G, zc, sizeof(T) == 8));
   unsigned nb = (unsigned)((int64_t)g.ntx * g.nty * g.nchunks);
@@ -1174,13 +1204,13 @@ bool launch_step_fused(Fields<const T> U, Fields<T> O, const Grid& G, const Step
   }
 #undef PMF_FUSED_RS
 #undef PMF_FUSED
-  hipLaunchKernelGGL(k_fold_max_flat, dim3(1), dim3(256), 0, st, red, (int)nb, dsmax);
+  if (dsmax) launch_fold_max(red, nb, dsmax, hsmax, st);
   return true;
 }
 
 bool launch_step_fused_surr(Fields<const float> U, Fields<float> O, const Grid& G, const StepParams<float>& P,
                             double* red, double* dsmax, const unsigned char* simg, float thr,
-                            unsigned long long* nsmooth, hipStream_t st) {
+                            unsigned long long* nsmooth, hipStream_t st, double* hsmax) {
   if (!surrogate_grid(G) || P.rsolve != RS_HLLD) return false;
   FusedGeom g = fused_geom(G, pick_zc(G, 2));
   unsigned nb = (unsigned)((int64_t)g.ntx * g.nty * g.nchunks);
@@ -1190,7 +1220,7 @@ bool launch_step_fused_surr(Fields<const float> U, Fields<float> O, const Grid& 
   else if (P.recon == RECON_PLM_MINMOD) PMF_FUSED_S(RECON_PLM_MINMOD);
   else PMF_FUSED_S(RECON_PLM);
 #undef PMF_FUSED_S
-  hipLaunchKernelGGL(k_fold_max_flat, dim3(1), dim3(256), 0, st, red, (int)nb, dsmax);
+  launch_fold_max(red, nb, dsmax, hsmax, st);
   return true;
 }
 
@@ -1486,9 +1516,9 @@ template bool launch_step_fused_ct<double>(Fields<const double>, Fields<double>,
 
 template bool launch_step_fused<float>(Fields<const float>, Fields<float>, const Grid&, const StepParams<float>&,
                                        double*, double*, hipStream_t, int, const SrcParams<float>*,
-                                       const StepParams<float>*);
+                                       const StepParams<float>*, double*);
 template bool launch_step_fused<double>(Fields<const double>, Fields<double>, const Grid&, const StepParams<double>&,
                                         double*, double*, hipStream_t, int, const SrcParams<double>*,
-                                        const StepParams<double>*);
+                                        const StepParams<double>*, double*);
 
 }  // namespace pmf

@@ -818,7 +818,7 @@ int pmf_step_surrogate(pmf_state* s, pmf_surrogate* n, double dt, double ch, dou
     mark(s);
     bool ok = launch_step_fused_surr(cfields_at<float>(s->U, s->nc), fields_at<float>(s->S, s->nc), s->G,
                                      make_params<float>(s, dt, ch, decay), s->red, s->dval, n->img, float(thr),
-                                     n->nsmooth, s->st);
+                                     n->nsmooth, s->st, s->hval);
     mark(s);
     if (!ok) throw Error("surrogate step unavailable for this configuration");
     hip_check(hipGetLastError(), "surrogate step launch");

@@ -120,6 +120,31 @@ void build_items(pmf_ensemble* e) {
   drop_graph(e);
 }
 
+// The plan before any tuning: a persistent workgroup for every place on the device (two per CU
+// left a third of them empty: 12.1 Mcells in 32 cubes 758 us a step, three 637), and the chunk
+// length, the same for all cubes, that fills them best (up to 16 planes: past that the last
+// items of the queues run long; 32: 668 us).
+void default_plan(pmf_ensemble* e) {
+  double best = 1e300;
+  int zc = 16;
+  int64_t items = 0;
+  for (int cand : {1, 2, 4, 8, 16}) {
+    int64_t groups = 0;
+    for (int n : e->edge) {
+      const FusedGeom g = ens_geom(n, std::min(cand, n));
+      groups += int64_t(g.ntx) * g.nty * g.nchunks;
+    }
+    const double c = fused_cost(groups, cand, 3);
+    if (c < best) {
+      best = c;
+      zc = cand;
+      items = groups;
+    }
+  }
+  for (int c = 0; c < e->ncubes; ++c) e->zc[c] = std::min(zc, e->edge[c]);
+  e->nwg = (int)std::min<int64_t>(fused_slots(), (items + 7) / 8 * 8);
+}
+
 void check_ens(const pmf_ensemble* e) {
   if (!e) throw Error("null ensemble");
 }
@@ -128,7 +153,8 @@ const Fields<float>& current(const pmf_ensemble* e, int c) { return e->parity ? 
 
 // One ensemble step on the stream: the per-cube CFL stage, then the persistent step.
 void enqueue_step(pmf_ensemble* e, int parity, float cfl, float fac, float cr) {
-  launch_ens_params(e->dcubes, e->ncubes, e->red, base_params(e), e->params, e->clock, e->ctr, cfl, fac, cr, e->st);
+  launch_ens_params(e->dcubes, e->ncubes, e->red, base_params(e), e->params, e->clock, e->ctr, e->nwg, cfl, fac, cr,
+                    e->st);
   launch_ens_step(e->dcubes, e->ditems, e->q, e->params, e->red, e->ctr, e->nwg, parity, e->p.recon, e->p.riemann,
                   e->st);
 }
@@ -170,7 +196,7 @@ int pmf_ensemble_create(const pmf_params* base, int32_t ncubes, const int32_t* e
       e->ncubes = ncubes;
       e->edge.assign(edge, edge + ncubes);
       e->zc.resize(ncubes);
-      for (int c = 0; c < ncubes; ++c) e->zc[c] = std::min(16, edge[c]);
+      default_plan(e);
       size_t total = 0;
       for (int c = 0; c < ncubes; ++c) total += size_t(18) * edge[c] * edge[c] * edge[c];
       hip_check(hipMalloc(&e->pool, sizeof(float) * total), "hipMalloc");
@@ -188,7 +214,7 @@ int pmf_ensemble_create(const pmf_params* base, int32_t ncubes, const int32_t* e
       hip_check(hipMalloc(&e->params, sizeof(StepParams<float>) * ncubes), "hipMalloc");
       hip_check(hipMalloc(&e->clock, sizeof(double) * 3 * ncubes), "hipMalloc");
       hip_check(hipMemset(e->clock, 0, sizeof(double) * 3 * ncubes), "hipMemset");
-      hip_check(hipMalloc(&e->ctr, sizeof(unsigned) * 8), "hipMalloc");
+      hip_check(hipMalloc(&e->ctr, sizeof(unsigned) * 8 * kEnsCtrStride), "hipMalloc");
       hip_check(hipStreamCreateWithFlags(&e->st, hipStreamNonBlocking), "hipStreamCreate");
       hip_check(hipEventCreate(&e->e0), "hipEventCreate");
       hip_check(hipEventCreate(&e->e1), "hipEventCreate");

@@ -62,6 +62,9 @@ bool launch_step_fused_surr(Fields<const float> U, Fields<float> O, const Grid& 
 // given precision with z chunks of zc planes (0 = the built-in choice).
 int64_t fused_blocks(const Grid& G, bool f64, int zc = 0);
 int fused_chunk(const Grid& G, bool f64);  // the built-in z chunk
+// Relative time of `groups` workgroups of zc planes each on this device, `slots` of them per CU.
+double fused_cost(int64_t groups, int zc, int slots);
+int fused_slots();  // float workgroups the device holds at once, a multiple of eight
 constexpr int kMinChunk = 4;  // smallest z chunk a caller may set (the built-in choice may be shorter)
 
 // Geometry of the fused kernel's work decomposition: 16x12 column tiles (x fastest,
@@ -81,19 +84,23 @@ struct EnsCube {
   double dx;
   int32_t item0, nitems;
 };
-// Eight work queues (one per XCD): contiguous slices [base, base + len) of the items.
+// Eight work queues (one per XCD): contiguous slices [base, base + len) of the items. Workgroup
+// b takes item b / 8 of queue b % 8 first; the counters, one to a cache line, hand out the
+// rest.
 struct EnsQueues {
   int32_t base[8], len[8];
 };
+constexpr int kEnsCtrStride = 32;  // unsigneds from one queue's counter to the next
 FusedGeom ens_geom(int n, int zc);
 // Initial CFL maxima, one per work item (items are (cube, tile) pairs).
 void launch_ens_wavespeed(const EnsCube* cubes, const int2* items, int nitems, const StepParams<float>& P,
                           double* red, int parity, hipStream_t st);
 // Per-cube dt / ch / decay from the item maxima in red; clock holds (t, dt, smax) per cube.
 void launch_ens_params(const EnsCube* cubes, int ncubes, const double* red, const StepParams<float>& base,
-                       StepParams<float>* params, double* clock, unsigned* ctr, float cfl, float fac, float cr,
+                       StepParams<float>* params, double* clock, unsigned* ctr, int nwg, float cfl, float fac, float cr,
                        hipStream_t st);
-// The persistent step over all items (nwg workgroups; ctr = eight queue counters).
+// The persistent step over all items (nwg workgroups, the same as launch_ens_params got; ctr =
+// eight queue counters).
 void launch_ens_step(const EnsCube* cubes, const int2* items, const EnsQueues& q, const StepParams<float>* params,
                      double* red, unsigned* ctr, int nwg, int parity, int recon, int rsolve, hipStream_t st);
 

@@ -1141,18 +1141,24 @@ static int device_cus() {
 // Measured (minmod, step and fold, the earlier rule's choice -> this one's): 16^3 23.7 -> 12.9
 // us (4 planes -> 1), 32^3 23.7 -> 13.6 (1), 64^3 31.4 -> 28.6 (2), 96^3 64 -> 55 (6); 128^3 (16)
 // and 256^3 (32) as before.
-static int pick_zc(const Grid& G, int slots) {
+double fused_cost(int64_t groups, int zc, int slots) {
   static const double kShare[2][4] = {{0, 1.0, 1.45, 1.45}, {0, 1.0, 1.19, 1.54}};
   const double* share = kShare[slots >= 3];
-  const int64_t tiles = (int64_t)((G.nx + TX - 1) / TX) * ((G.ny + TY - 1) / TY);
   const int64_t cus = device_cus();
+  const int64_t full = groups / (slots * cus), rest = groups - full * slots * cus;
+  return (double(full) * share[slots] + share[(rest + cus - 1) / cus]) * (zc + 2);
+}
+
+int fused_slots() { return 3 * device_cus() / 8 * 8; }
+
+static int pick_zc(const Grid& G, int slots) {
+  const int64_t tiles = (int64_t)((G.nx + TX - 1) / TX) * ((G.ny + TY - 1) / TY);
   int best = 1;
   double cost = 1e300;
   for (int zc = 1; zc <= 32 && zc <= G.nz; ++zc) {
     const int chunks = (G.nz + zc - 1) / zc;
     if (zc > 1 && (G.nz + chunks - 1) / chunks != zc) continue;  // a shorter chunk gives as many
-    const int64_t groups = tiles * chunks, full = groups / (slots * cus), rest = groups - full * slots * cus;
-    const double c = (double(full) * share[slots] + share[(rest + cus - 1) / cus]) * (zc + 2);
+    const double c = fused_cost(tiles * chunks, zc, slots);
     if (c < cost) {
       cost = c;
       best = zc;
@@ -1264,11 +1270,12 @@ __global__ __launch_bounds__(FTHREADS) void k_ens_wavespeed(const EnsCube* __res
 // Per-cube CFL stage (timestep.jl:39 and driver.jl:48-71 in float32 arithmetic, the same
 // operations as the single-state host path): fold the cube's item maxima, then
 // dt = cfl dx / max(smax, eps), ch = glm_ch_fac smax, dt_used = dt smax / max(smax, ch),
-// decay = exp(-cr ch dt_used / dx). Also clears the step's work queues.
+// decay = exp(-cr ch dt_used / dx). Also sets the step's work queues past the items that the
+// workgroups take first.
 __global__ __launch_bounds__(256) void k_ens_params(const EnsCube* __restrict__ cubes, const double* __restrict__ red,
                                                     StepParams<float> base, StepParams<float>* __restrict__ params,
-                                                    double* __restrict__ clock, unsigned* __restrict__ ctr, float cfl,
-                                                    float fac, float cr) {
+                                                    double* __restrict__ clock, unsigned* __restrict__ ctr,
+                                                    unsigned first, float cfl, float fac, float cr) {
   __shared__ double sh[4];
   const int c = blockIdx.x;
   const EnsCube& cb = cubes[c];
@@ -1299,7 +1306,7 @@ __global__ __launch_bounds__(256) void k_ens_params(const EnsCube* __restrict__ 
     clock[3 * c + 1] = dtf;
     clock[3 * c + 2] = smax;
     if (c == 0) {
-      for (int q = 0; q < 8; ++q) ctr[q] = 0u;
+      for (int q = 0; q < 8; ++q) ctr[q * kEnsCtrStride] = first;
     }
   }
 }
@@ -1314,17 +1321,29 @@ __device__ __forceinline__ void ens_step_body(const EnsCube* __restrict__ cubes,
   unsigned none = 0;
   int qi = 0;  // queues tried so far (thread 0)
   const int home = blockIdx.x & 7;
-  for (;;) {
+  const int first = gridDim.x >> 3;  // items of each queue that its own workgroups take without asking
+  for (bool start = true;; start = false) {
     if (threadIdx.x == 0) {
       int got = -1;
-      while (qi < 8) {
-        const int qq = (home + qi) & 7;
-        const unsigned k = atomicAdd(&ctr[qq], 1u);
-        if (k < (unsigned)q.len[qq]) {
-          got = q.base[qq] + (int)k;
-          break;
+      if (start && (int)(blockIdx.x >> 3) < q.len[home]) {
+        got = q.base[home] + (int)(blockIdx.x >> 3);
+      } else {
+        // a queue is asked (an atomic add that all idle workgroups would queue for) only while its
+        // counter shows items left: with one add per workgroup and queue on one cache line a step
+        // of eight 16^3 cubes took 40 us at 256 workgroups and 105 at 1024, now 20 at either; of
+        // four 32^3 and two 64^3 95, now 58
+        for (; qi < 8; ++qi) {
+          const int qq = (home + qi) & 7;
+          unsigned* c = &ctr[qq * kEnsCtrStride];
+          if (q.len[qq] <= first ||
+              __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= (unsigned)q.len[qq])
+            continue;
+          const unsigned k = atomicAdd(c, 1u);
+          if (k < (unsigned)q.len[qq]) {
+            got = q.base[qq] + (int)k;
+            break;
+          }
         }
-        ++qi;
       }
       sItem = got;
     }
@@ -1378,10 +1397,10 @@ void launch_ens_wavespeed(const EnsCube* cubes, const int2* items, int nitems, c
 }
 
 void launch_ens_params(const EnsCube* cubes, int ncubes, const double* red, const StepParams<float>& base,
-                       StepParams<float>* params, double* clock, unsigned* ctr, float cfl, float fac, float cr,
+                       StepParams<float>* params, double* clock, unsigned* ctr, int nwg, float cfl, float fac, float cr,
                        hipStream_t st) {
-  hipLaunchKernelGGL(k_ens_params, dim3(ncubes), dim3(256), 0, st, cubes, red, base, params, clock, ctr, cfl, fac,
-                     cr);
+  hipLaunchKernelGGL(k_ens_params, dim3(ncubes), dim3(256), 0, st, cubes, red, base, params, clock, ctr,
+                     (unsigned)nwg >> 3, cfl, fac, cr);
 }
 
 void launch_ens_step(const EnsCube* cubes, const int2* items, const EnsQueues& q, const StepParams<float>* params,

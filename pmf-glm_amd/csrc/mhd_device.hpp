@@ -11,6 +11,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace pmf {
 
 enum { RECON_PLM = 0, RECON_PPM = 1, RECON_PLM_MINMOD = 2 };
@@ -79,6 +81,26 @@ __device__ __forceinline__ double dfma(double a, double b, double c) { return __
 __device__ __forceinline__ float dcopysign(float a, float b) { return __builtin_copysignf(a, b); }
 __device__ __forceinline__ double dcopysign(double a, double b) { return __builtin_copysign(a, b); }
 __device__ __forceinline__ double dabs(double a) { return __builtin_fabs(a); }
+
+// XCD-aware tile order: dispatch round-robins workgroups over the 8 XCDs, so XCD x gets
+// workgroups x, x + 8, ...; they take a contiguous range of tiles (nwg / 8, one more for the
+// first nwg % 8 XCDs), whose halo re-reads its L2 then serves.
+__device__ __forceinline__ int xcd_tile() {
+  const int nwg = gridDim.x, x = blockIdx.x & 7;
+  return x * (nwg >> 3) + min(x, nwg & 7) + (blockIdx.x >> 3);
+}
+
+// Address of cell idx of one field. NARROW: the byte offset fits 32 bits (fields below
+// 4 GiB), so every access is the field's scalar base plus one 32-bit vector offset shared
+// by the nine fields (global_load/store with saddr) instead of a 64-bit address each.
+template <bool NARROW, class T> __device__ __forceinline__ T* cell_at(T* base, int64_t idx) {
+  if constexpr (NARROW) {
+    using B = typename std::conditional<std::is_const<T>::value, const char, char>::type;
+    return reinterpret_cast<T*>(reinterpret_cast<B*>(base) + (uint32_t)idx * (uint32_t)sizeof(T));
+  } else {
+    return base + idx;
+  }
+}
 
 // cons2prim (glm_physics.jl:11-18): density floored before the velocity and kinetic
 // energy, pressure floored at pfl.

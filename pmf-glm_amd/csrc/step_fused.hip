@@ -66,18 +66,6 @@ __device__ __forceinline__ int src_index(int i, int n, int bc, bool& flip) {
   return min(max(r, 0), n - 1);
 }
 
-// Address of cell idx of one field. NARROW: the byte offset fits 32 bits (fields below
-// 4 GiB), so every access is the field's scalar base plus one 32-bit vector offset shared
-// by the nine fields (global_load/store with saddr) instead of a 64-bit address each.
-template <bool NARROW, class T> __device__ __forceinline__ T* cell_at(T* base, int64_t idx) {
-  if constexpr (NARROW) {
-    using B = typename std::conditional<std::is_const<T>::value, const char, char>::type;
-    return reinterpret_cast<T*>(reinterpret_cast<B*>(base) + (uint32_t)idx * (uint32_t)sizeof(T));
-  } else {
-    return base + idx;
-  }
-}
-
 template <bool NARROW, class T>
 __device__ __forceinline__ void load_cons(const Fields<const T>& U, int64_t idx, T* c) {
 #pragma unroll
@@ -564,12 +552,26 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
           Rz[v] = mh[v] + dLz[v];
           Lzn[v] = mh[v] + dRz[v];
         }
-        src_face_pre(fx, m0, dRx, src, cv);
-        src_face_pre(fy, m0, dRy, src, cv);
-        src_face_pre(Rx, m0, dLx, src, cv);
-        src_face_pre(Ry, m0, dLy, src, cv);
-        src_face_pre(Rz, m0, dLz, src, cv);
-        src_face_pre(Lzn, m0, dRz, src, cv);
+        if constexpr (CT) {  // the form whose bits the edge upwinding was pinned with
+          src_face_pre(fx, m0, dRx, src, cv);
+          src_face_pre(fy, m0, dRy, src, cv);
+          src_face_pre(Rx, m0, dLx, src, cv);
+          src_face_pre(Ry, m0, dLy, src, cv);
+          src_face_pre(Rz, m0, dLz, src, cv);
+          src_face_pre(Lzn, m0, dRz, src, cv);
+        } else {
+          T base[3], slope;
+          src_base(m0, mh, src, cv, base, slope);
+#pragma unroll
+          for (int c = 0; c < 3; ++c) {
+            fx[1 + c] = dfma(slope, dRx[1 + c], base[c]);
+            fy[1 + c] = dfma(slope, dRy[1 + c], base[c]);
+            Rx[1 + c] = dfma(slope, dLx[1 + c], base[c]);
+            Ry[1 + c] = dfma(slope, dLy[1 + c], base[c]);
+            Rz[1 + c] = dfma(slope, dLz[1 + c], base[c]);
+            Lzn[1 + c] = dfma(slope, dRz[1 + c], base[c]);
+          }
+        }
         if (xleft) {
 #pragma unroll
           for (int v = 0; v < 9; ++v) S.sLX[v * NFX + xl(ix, iy)] = fx[v];
@@ -847,14 +849,6 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
   return smax;
 }
 
-// XCD-aware tile order: dispatch round-robins workgroups over the 8 XCDs, so XCD x gets
-// workgroups x, x + 8, ...; they take a contiguous range of tiles (nwg / 8, one more for the
-// first nwg % 8 XCDs), whose halo re-reads its L2 then serves.
-__device__ __forceinline__ int xcd_tile() {
-  const int nwg = gridDim.x, x = blockIdx.x & 7;
-  return x * (nwg >> 3) + min(x, nwg & 7) + (blockIdx.x >> 3);
-}
-
 // Block-wide CFL maximum of the threads' running maxima, stored by thread 0.
 template <class T>
 __device__ __forceinline__ void block_store_max(T smax, T* sMax, double* out) {
@@ -872,10 +866,9 @@ __device__ __forceinline__ void block_store_max(T smax, T* sMax, double* out) {
 
 // Three waves per SIMD (168 VGPRs; three 38 KB workgroups then share a CU's LDS) for
 // every plain float variant and the PLM source variants. PLM fits the plain step without
-// spilling; PPM keeps both edge offsets of each direction live and is still faster at
-// three waves than at two. The PLM source variants (drag, radiation) spill 4-7 dwords at
-// three waves and run 14-17% faster than at two; the PPM source variants would spill 44
-// and keep the compiler's default (two waves).
+// spilling, the PLM source variants (drag, radiation) among them; PPM keeps both edge offsets
+// of each direction live and is still faster at three waves than at two. The PPM source
+// variants would spill 44 and keep the compiler's default (two waves).
 template <class T, int RECON, int RS, bool SURR, bool SRC>
 constexpr bool fused_three_waves() {
   return sizeof(T) == 4 && !SURR && !(SRC && RECON == RECON_PPM);

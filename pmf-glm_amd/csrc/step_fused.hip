@@ -175,7 +175,7 @@ struct FusedLds {
 // thread's running CFL maximum of the cells it stored. SURR: the surrogate-assisted
 // variant (float only): each face is gated by the jump detector and solved by the
 // learned flux (wave-level MFMA) or by HLLD; sW holds the network's LDS image
-// (surrogate.hpp), sB its biases (global memory), and smooth_count counts the faces that
+// (surrogate.hpp), and smooth_count counts the faces that
 // used it (each face once, as the lower face of its cell).
 // Cell EMF -v x B (integrator_ref.jl:133-138) from the predicted velocity v and the
 // start-of-step field b (primitive slots), without contraction, so that the step's two
@@ -195,8 +195,7 @@ template <class T, int RECON, int RS, bool SURR, bool SRC = false, bool NARROW =
 __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T>& O, const FusedGeom& g,
                                         const StepParams<T>& P, int w,
                                         FusedLds<T, SRC, dxy_in_lds<RECON, SURR>(), EDGES>& S,
-                                        const unsigned short* __restrict__ sW, const float* __restrict__ sB,
-                                        float thr, unsigned& smooth_count, const SrcParams<T>& src,
+                                        const unsigned short* sW, float thr, unsigned& smooth_count, const SrcParams<T>& src,
                                         SurrQueue<FQCAP>* Qp = nullptr, T* __restrict__ ctp = nullptr) {
   static_assert(!(CT && SURR), "the fused CT step has no surrogate");
   static_assert(!(BCG && (CT || SURR)), "the CT and surrogate steps run on periodic grids");
@@ -718,7 +717,7 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
       }
       __syncthreads();
       const int nq = (int)Q.n;
-      for (int b = (t >> 6) * 32; b < nq; b += FTHREADS / 2) surr_batch(b, nq, Q, sW, sB);
+      for (int b = (t >> 6) * 32; b < nq; b += FTHREADS / 2) surr_batch(b, nq, Q, sW);
       __syncthreads();
       float y[SURR_OUT];
       if (stores) {
@@ -893,22 +892,19 @@ __device__ __forceinline__ void step_fused_body(const Fields<const T>& U, const 
                                                 unsigned long long* __restrict__ nsmooth, const SrcParams<T>& src) {
   __shared__ FusedLds<T, SRC, dxy_in_lds<RECON, SURR>()> lds;
   __shared__ T sMax[FTHREADS / 64];
-  __shared__ __attribute__((aligned(16))) unsigned short sW[SURR ? SIMG_NW : 2];
+  __shared__ __attribute__((aligned(16))) unsigned short sW[SURR ? SIMG_BYTES / 2 : 2];
   __shared__ __attribute__((aligned(16))) SurrQueue<SURR ? FQCAP : 1> sQ;
   unsigned smooth_count = 0;
   if constexpr (SURR) {
     const unsigned* src = reinterpret_cast<const unsigned*>(simg);
     unsigned* dw = reinterpret_cast<unsigned*>(sW);
-    for (int e = threadIdx.x; e < SIMG_NW / 2; e += FTHREADS) dw[e] = src[e];
+    for (int e = threadIdx.x; e < SIMG_BYTES / 4; e += FTHREADS) dw[e] = src[e];
   }
   const int w = xcd_tile();
   SurrQueue<FQCAP>* q = nullptr;
   if constexpr (SURR) q = &sQ;
-  // the biases (the image's float tail) stay in global memory: with them out of LDS the
-  // surrogate step's 81.6 KB lets two workgroups share a CU
-  const float* sB = SURR ? reinterpret_cast<const float*>(simg + SIMG_NW * 2) : nullptr;
   const T smax =
-      fused_item<T, RECON, RS, SURR, SRC, NARROW, false, BCG>(U, O, g, P, w, lds, sW, sB, thr, smooth_count, src, q);
+      fused_item<T, RECON, RS, SURR, SRC, NARROW, false, BCG>(U, O, g, P, w, lds, sW, thr, smooth_count, src, q);
   // fold the workgroup's CFL maximum (timestep.jl:8-12 on the new state)
   block_store_max(smax, sMax, red + blockIdx.x);
   if constexpr (SURR) {
@@ -940,7 +936,7 @@ __global__ __launch_bounds__(FTHREADS) __attribute__((amdgpu_waves_per_eu(3))) v
 }
 
 // Two waves per SIMD. The surrogate-assisted step: about 250 VGPRs with the network in its
-// own function and 81.6 KB of LDS, so two workgroups share a CU and one's network batches
+// own function and 79.4 KB of LDS, so two workgroups share a CU and one's network batches
 // overlap the other's HLLD faces and barriers. float64 PLM: 76 KB of LDS, two workgroups.
 template <class T, int RECON, int RS, bool SURR, bool SRC, bool NARROW, bool BCG>
 __global__ __launch_bounds__(FTHREADS) __attribute__((amdgpu_waves_per_eu(2))) void k_step_fused2(
@@ -1353,7 +1349,7 @@ __device__ __forceinline__ void ens_step_body(const EnsCube* __restrict__ cubes,
     for (int v = 0; v < 9; ++v) U.v[v] = in.v[v];
     const StepParams<float> P = params[c];
     const float smax =
-        fused_item<float, RECON, RS, false, false, true>(U, out, cb.g, P, w, lds, nullptr, nullptr, 0.f, none,
+        fused_item<float, RECON, RS, false, false, true>(U, out, cb.g, P, w, lds, nullptr, 0.f, none,
                                                          SrcParams<float>{});
     block_store_max(smax, sMax, red + i);
     __syncthreads();  // sItem and sMax are reused by the next item
@@ -1430,7 +1426,7 @@ __device__ __forceinline__ void step_fused_ct_body(const Fields<const T>& U, con
   __shared__ FusedLds<T, SRC, dxy_in_lds<RECON, false>(), EDGES> lds;
   const int w = xcd_tile();
   unsigned none = 0;
-  (void)fused_item<T, RECON, RS, false, SRC, NARROW, true, false, EDGES>(U, O, g, P, w, lds, nullptr, nullptr, 0.f,
+  (void)fused_item<T, RECON, RS, false, SRC, NARROW, true, false, EDGES>(U, O, g, P, w, lds, nullptr, 0.f,
                                                                          none, src, nullptr, ctp);
 }
 

@@ -130,16 +130,17 @@ __device__ __forceinline__ float bf16_round(float f) {
 namespace pmf {
 
 // LDS image of the network for wave-level inference: transposed weights W_l^T [out][in]
-// in bfloat16 with rows padded by 4 (bank spread, 8-byte aligned MFMA A fragments), the
-// output layer padded to 32 rows, then the float32 biases.
+// in bfloat16 with rows padded by 4 (bank spread, 8-byte aligned MFMA A fragments), then the
+// float32 biases (the output layer's padded to 32).
 constexpr int SIMG_S1 = 16 + 4, SIMG_S2 = 64 + 4;
 constexpr int SIMG_W1 = 0;                       // 64 x 20
 constexpr int SIMG_W2 = SIMG_W1 + 64 * SIMG_S1;  // 64 x 68
 constexpr int SIMG_W3 = SIMG_W2 + 64 * SIMG_S2;  // 64 x 68
-constexpr int SIMG_W4 = SIMG_W3 + 64 * SIMG_S2;  // 32 x 68
-constexpr int SIMG_NW = SIMG_W4 + 32 * SIMG_S2;  // bf16 entries: 12160
+constexpr int SIMG_W4 = SIMG_W3 + 64 * SIMG_S2;  // 9 x 68
+constexpr int SIMG_NW = SIMG_W4 + SURR_OUT * SIMG_S2 + 4;  // bf16 entries, to a multiple of 16 bytes: 10600
 constexpr int SIMG_NB = 64 * 3 + 32;             // float biases (output padded)
 constexpr int SIMG_BYTES = SIMG_NW * 2 + SIMG_NB * 4;
+static_assert(SIMG_NW * 2 % 16 == 0 && SIMG_W4 % 4 == 0, "aligned fragments and biases");
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
@@ -161,76 +162,17 @@ __device__ __forceinline__ bf16x8 lds_frag8(const unsigned short* row, int c0, i
 
 // Accumulator initialised with the layer's biases: register r of lane half h holds unit
 // 32 mb + 8 (r / 4) + 4 h + r % 4 (the 32x32 MFMA output layout).
-__device__ __forceinline__ sf32x16 bias_acc(const float* __restrict__ b, int mb, int lh) {
+__device__ __forceinline__ sf32x16 bias_acc(const float* b, int mb, int lh) {
   sf32x16 d;
 #pragma unroll
-  for (int r = 0; r < 16; ++r) d[r] = b[32 * mb + 8 * (r / 4) + 4 * lh + r % 4];
-  return d;
-}
-
-// y[9] = MLP(x[16]) for the 64 faces held by the 64 lanes of the calling wave (one face
-// per lane). Must be called by all lanes of the wave. Units are the MFMA rows and faces
-// the columns (32 per pass); v_mfma_f32_32x32x16_bf16 contracts 16 units per step. The
-// hidden layers' contraction order is permuted so that accumulator registers 8s..8s+7
-// of a lane are exactly its B fragment for step s of the next layer (lane half h then
-// holds units 16s + 4h + {0..3} and 16s + 8 + 4h + {0..3}); the weight fragments read
-// the same units. Activations never leave registers.
-// npass = 1 evaluates only the faces of lanes 0-31 (results in lanes 0-31).
-__device__ inline __attribute__((noinline)) void mlp_wave(const float* x, float* y,
-                                                        const unsigned short* __restrict__ sw,
-                                                        const float* __restrict__ sb, int npass = 2) {
-  const int lane = threadIdx.x & 63, li = lane & 31, lh = lane >> 5;
-#pragma unroll 1
-  for (int pass = 0; pass < npass; ++pass) {
-    const int src = pass * 32 + li;
-    // layer 1: inputs 8h..8h+7 of face (pass, li) in lane half h
-    bf16x8 bin;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const float lo = __shfl(x[q], src, 64), hi = __shfl(x[8 + q], src, 64);
-      bin[q] = (__bf16)(lh ? hi : lo);
-    }
-    sf32x16 d[2];
-#pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
-      d[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-          lds_frag8(sw + SIMG_W1 + (mb * 32 + li) * SIMG_S1, 8 * lh, 8 * lh + 4), bin, bias_acc(sb, mb, lh), 0, 0, 0);
-#pragma unroll 1
-    for (int layer = 1; layer < 4; ++layer) {
-      bf16x8 b[4];
-#pragma unroll
-      for (int st = 0; st < 4; ++st)
-#pragma unroll
-        for (int q = 0; q < 8; ++q) b[st][q] = (__bf16)gelu(d[st >> 1][8 * (st & 1) + q]);
-      const int off = layer == 1 ? SIMG_W2 : layer == 2 ? SIMG_W3 : SIMG_W4;
-      const int nmb = layer == 3 ? 1 : 2;
-      const float* bias = sb + 64 * layer;
-#pragma unroll
-      for (int mb = 0; mb < 2; ++mb) {
-        if (mb >= nmb) break;
-        sf32x16 acc = bias_acc(bias, mb, lh);
-        const unsigned short* row = sw + off + (mb * 32 + li) * SIMG_S2;
-#pragma unroll
-        for (int st = 0; st < 4; ++st)
-          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lds_frag8(row, 16 * st + 4 * lh, 16 * st + 8 + 4 * lh), b[st],
-                                                         acc, 0, 0, 0);
-        d[mb] = acc;
-      }
-    }
-    // outputs o of face column j: o = 0..3 in lane j (registers 0..3), o = 4..7 in lane
-    // j+32 (registers 0..3), o = 8 in lane j (register 4)
-    float o[9];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      o[q] = __shfl(d[0][q], li, 64);
-      o[4 + q] = __shfl(d[0][q], li + 32, 64);
-    }
-    o[8] = __shfl(d[0][4], li, 64);
-    if (lh == pass) {
-#pragma unroll
-      for (int k = 0; k < 9; ++k) y[k] = o[k];
-    }
+  for (int r = 0; r < 4; ++r) {
+    const float4 v = *reinterpret_cast<const float4*>(b + 32 * mb + 8 * r + 4 * lh);
+    d[4 * r] = v.x;
+    d[4 * r + 1] = v.y;
+    d[4 * r + 2] = v.z;
+    d[4 * r + 3] = v.w;
   }
+  return d;
 }
 
 }  // namespace pmf
@@ -322,35 +264,69 @@ __device__ __forceinline__ int surr_enqueue(bool want, const float* x, SurrQueue
   return slot;
 }
 
-// One batch of up to 32 queued faces (slots b .. b+31 below nq, one MFMA pass), evaluated
-// by the calling wave (lanes 0-31 hold the faces); all lanes of the wave must call it.
+// One batch of up to 32 queued faces (slots b .. b+31 below nq), evaluated by the calling wave;
+// all its lanes must call it. img: the network's image, in LDS. Units are the MFMA rows and
+// faces the columns; v_mfma_f32_32x32x16_bf16 contracts 16 units per step. A slot's 32 bytes
+// are the two lane halves' B fragments of the first layer as they stand; the hidden layers'
+// contraction order is permuted so that accumulator registers 8s..8s+7 of a lane are its B
+// fragment for step s of the next layer (lane half h then holds units 16s + 4h + {0..3} and
+// 16s + 8 + 4h + {0..3}; the weight fragments read the same units); and the outputs leave from
+// the registers they arrive in (lane half 0: 0..3, half 1: 4..7, 5 not learned). So
+// activations never leave registers and no lane exchanges anything. The two accumulators'
+// chains alternate and a layer's weights are read before the activations that they wait for.
+// Bound: the 96 GELUs a lane (two quarter-rate and five full-rate operations each) at two
+// waves per SIMD. Through arrays in scratch memory, lane shuffles, biases in global memory
+// and one accumulator after the other a 192^3 step with 0.90 / 0.31 / 0.11 of its faces in the
+// network took 2.71 / 1.53 / 1.11 ms, now 2.19 / 1.31 / 0.99. A function of its own, for one
+// batch: inlined, with the loop inside, or for two batches at once its registers push the
+// step's own carries into scratch (a step without network faces 0.56 -> 1.39 / 0.64 / 1.07 ms).
 template <int CAP>
-__device__ __forceinline__ void surr_batch(int b, int nq, SurrQueue<CAP>& Q, const unsigned short* __restrict__ sw,
-                                           const float* __restrict__ sb) {
-  const int lane = threadIdx.x & 63;
-  const int slot = b + lane;
-  const bool valid = lane < 32 && slot < nq;
-  float x[SURR_IN];
-  if (valid) {
-    const uint4 a = Q.slot[2 * slot];
-    const uint4 c = Q.slot[2 * slot + 1];
-    const unsigned w[8] = {a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
+__device__ __attribute__((noinline)) void surr_batch(int b, int nq, SurrQueue<CAP>& Q, const unsigned short* img) {
+  const int lane = threadIdx.x & 63, li = lane & 31, lh = lane >> 5;
+  const float* bias = reinterpret_cast<const float*>(img + SIMG_NW);
+  const int slot = min(b + li, nq - 1);  // lanes past the end repeat the last face
+  bf16x8 w[2][4], f[4];
+  f[0] = __builtin_bit_cast(bf16x8, Q.slot[2 * slot + lh]);
+  sf32x16 d[2];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      x[2 * k] = __builtin_bit_cast(float, w[k] << 16);
-      x[2 * k + 1] = __builtin_bit_cast(float, w[k] & 0xffff0000u);
-    }
-  } else {
+  for (int mb = 0; mb < 2; ++mb)
+    d[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+        lds_frag8(img + SIMG_W1 + (mb * 32 + li) * SIMG_S1, 8 * lh, 8 * lh + 4), f[0], bias_acc(bias, mb, lh), 0, 0, 0);
+#pragma unroll 1
+  for (int layer = 1; layer < 3; ++layer) {
+    const unsigned short* row = img + (layer == 1 ? SIMG_W2 : SIMG_W3) + li * SIMG_S2;
 #pragma unroll
-    for (int k = 0; k < SURR_IN; ++k) x[k] = 0.f;
+    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+      for (int st = 0; st < 4; ++st)
+        w[mb][st] = lds_frag8(row + mb * 32 * SIMG_S2, 16 * st + 4 * lh, 16 * st + 8 + 4 * lh);
+#pragma unroll
+    for (int st = 0; st < 4; ++st)
+#pragma unroll
+      for (int q = 0; q < 8; ++q) f[st][q] = (__bf16)gelu(d[st >> 1][8 * (st & 1) + q]);
+    d[0] = bias_acc(bias + 64 * layer, 0, lh);
+    d[1] = bias_acc(bias + 64 * layer, 1, lh);
+#pragma unroll
+    for (int st = 0; st < 4; ++st)
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb) d[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[mb][st], f[st], d[mb], 0, 0, 0);
   }
-  float y[SURR_OUT];
-  mlp_wave(x, y, sw, sb, 1);
-  // the slot's inputs were read above by this lane, the only one that touches the slot
-  if (valid) {
-    float* out = reinterpret_cast<float*>(&Q.slot[2 * slot]);
+  // output layer: rows past the nine outputs are never read
+  const unsigned short* row = img + SIMG_W4 + min(li, SURR_OUT - 1) * SIMG_S2;
 #pragma unroll
-    for (int j = 0; j < SURR_QOUT; ++j) out[j] = y[surr_qk(j)];
+  for (int st = 0; st < 4; ++st) w[0][st] = lds_frag8(row, 16 * st + 4 * lh, 16 * st + 8 + 4 * lh);
+#pragma unroll
+  for (int st = 0; st < 4; ++st)
+#pragma unroll
+    for (int q = 0; q < 8; ++q) f[st][q] = (__bf16)gelu(d[st >> 1][8 * (st & 1) + q]);
+  sf32x16 o = bias_acc(bias + 192, 0, lh);
+#pragma unroll
+  for (int st = 0; st < 4; ++st) o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[0][st], f[st], o, 0, 0, 0);
+  // the slots' inputs were read above by this wave, the only one that touches them
+  if (b + li < nq) {
+    float4 v = make_float4(o[0], o[1], o[2], o[3]);
+    if (lh) v = make_float4(o[0], o[2], o[3], 0.f);
+    *reinterpret_cast<float4*>(&Q.slot[2 * slot + lh]) = v;
   }
 }
 

@@ -66,10 +66,13 @@ __device__ __forceinline__ int src_index(int i, int n, int bc, bool& flip) {
   return min(max(r, 0), n - 1);
 }
 
-template <bool NARROW, class T>
+// The first N of the nine fields; the others come back zero.
+template <bool NARROW, int N, class T>
 __device__ __forceinline__ void load_cons(const Fields<const T>& U, int64_t idx, T* c) {
 #pragma unroll
-  for (int v = 0; v < 9; ++v) c[v] = *cell_at<NARROW>(U.v[v], idx);
+  for (int v = 0; v < N; ++v) c[v] = *cell_at<NARROW>(U.v[v], idx);
+#pragma unroll
+  for (int v = N; v < 9; ++v) c[v] = T(0);
 }
 
 // Ring cell h (0..NRING-1) at distance r from the tile: bottom row, top row, left
@@ -158,12 +161,14 @@ constexpr bool dxy_in_lds() {
 // predicted region are exchanged through LDS.
 constexpr int FNFXE = (TX + 1) * (TY + 1);  // x faces of rows -1..TY-1: 221
 constexpr int FNFYE = (TX + 1) * (TY + 1);  // y faces of columns -1..TX-1: 221
-template <class T, bool SRC = false, bool DXL = true, bool EDGES = false>
+// CT: eight fields (no psi), and without sources five updated components.
+template <class T, bool SRC = false, bool DXL = true, bool EDGES = false, bool CT = false>
 struct FusedLds {
-  T sP[2][9 * FNP];  // primitive planes m (current) and m-1, alternating
-  T sLX[9 * (EDGES ? FNFXE : FNFX)];  // left states of the x faces, then the x-face fluxes
-  T sLY[9 * (EDGES ? FNFYE : FNFY)];  // left states of the y faces, then the y-face fluxes
-  T sD[DXL ? 9 * NOWN : 1];  // DXL: each owned column's x/y divergence, carried a plane
+  static constexpr int NV = CT ? 8 : 9, ND = CT ? (SRC ? 8 : 5) : 9;
+  T sP[2][NV * FNP];  // primitive planes m (current) and m-1, alternating
+  T sLX[NV * (EDGES ? FNFXE : FNFX)];  // left states of the x faces, then the x-face fluxes
+  T sLY[NV * (EDGES ? FNFYE : FNFY)];  // left states of the y faces, then the y-face fluxes
+  T sD[DXL ? ND * NOWN : 1];  // DXL: each owned column's x/y divergence, carried a plane
   unsigned char sMk[SRC ? FNQ : 1];  // masked-fallback flags of the predicted cells
   T sZf[EDGES ? 3 * FNQ : 1];        // EDGES: mass, Bx and By fluxes of the z face m-1/2
   T sEz[EDGES ? FNQ : 1];            // EDGES: cell EMF z of plane m
@@ -194,12 +199,22 @@ template <class T, int RECON, int RS, bool SURR, bool SRC = false, bool NARROW =
           bool BCG = false, bool EDGES = false>
 __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T>& O, const FusedGeom& g,
                                         const StepParams<T>& P, int w,
-                                        FusedLds<T, SRC, dxy_in_lds<RECON, SURR>(), EDGES>& S,
+                                        FusedLds<T, SRC, dxy_in_lds<RECON, SURR>(), EDGES, CT>& S,
                                         const unsigned short* sW, float thr, unsigned& smooth_count, const SrcParams<T>& src,
                                         SurrQueue<FQCAP>* Qp = nullptr, T* __restrict__ ctp = nullptr) {
   static_assert(!(CT && SURR), "the fused CT step has no surrogate");
   static_assert(!(BCG && (CT || SURR)), "the CT and surrogate steps run on periodic grids");
   static_assert(!EDGES || (CT && !SRC), "edge EMFs belong to the plain CT step");
+  // Under CT psi takes no part (its flux is zero and the step clears it), the normal field of a
+  // face state is the face field, and cell B is the face average after the step, so its
+  // update is left out unless the sources' energy floor reads it. NV: fields that are loaded
+  // and predicted; ND: components updated from the fluxes; and by component, whether the x / y
+  // left states and fluxes go through LDS.
+  constexpr int NV = CT ? 8 : 9, ND = CT ? (SRC ? 8 : 5) : 9;
+  auto xstate = [](int v) { return !CT || (v != 5 && v != 8); };
+  auto ystate = [](int v) { return !CT || (v != 6 && v != 8); };
+  auto xflux = [](int v) { return v < ND || (EDGES && (v == 6 || v == 7)); };
+  auto yflux = [](int v) { return v < ND || (EDGES && (v == 5 || v == 7)); };
   const int tx = w % g.ntx;
   const int ty = (w / g.ntx) % g.nty;
   const int chunk = w / (g.ntx * g.nty);
@@ -245,14 +260,14 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
       bool fz = false;
       int kz = z;
       if (z < 0 || z >= g.nz) kz = src_index(z, g.nz, g.bc[2], fz);
-      load_cons<NARROW>(U, (int64_t)kz * g.plane + c2, c);
+      load_cons<NARROW, NV>(U, (int64_t)kz * g.plane + c2, c);
       const int f = (flips >> sh) & 3;
       if (f & 1) { c[1] = -c[1]; c[5] = -c[5]; }
       if (f & 2) { c[2] = -c[2]; c[6] = -c[6]; }
       if (fz) { c[3] = -c[3]; c[7] = -c[7]; }
     } else {
       (void)sh;
-      load_cons<NARROW>(U, (int64_t)wrapi(z, g.nz) * g.plane + c2, c);
+      load_cons<NARROW, NV>(U, (int64_t)wrapi(z, g.nz) * g.plane + c2, c);
     }
   };
   const bool xsolver = has_col && iy >= 0 && iy < vy && ix >= 0 && ix <= vx;  // owned + right ring column
@@ -299,11 +314,11 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
       load_plane(z0 - 2, col, 0, c);
       cons2prim(c, q, P);
 #pragma unroll
-      for (int v = 0; v < 9; ++v) S.sP[(z0 - 2) & 1][v * FNP + me] = q[v];
+      for (int v = 0; v < NV; ++v) S.sP[(z0 - 2) & 1][v * FNP + me] = q[v];
       load_plane(z0 - 1, col, 0, c);
       cons2prim(c, q, P);
 #pragma unroll
-      for (int v = 0; v < 9; ++v) S.sP[(z0 - 1) & 1][v * FNP + me] = q[v];
+      for (int v = 0; v < NV; ++v) S.sP[(z0 - 1) & 1][v * FNP + me] = q[v];
     }
     // EDGES: ring row -1 and column -1 are predicted on the chunk's first plane as well,
     // so that plane's extra cells (their slopes' second neighbours) are needed too
@@ -311,14 +326,14 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
       load_plane(z0 - 1, ecol, 2, c);
       cons2prim(c, q, P);
 #pragma unroll
-      for (int v = 0; v < 9; ++v) S.sP[(z0 - 1) & 1][v * FNP + pidx(ex, ey)] = q[v];
+      for (int v = 0; v < NV; ++v) S.sP[(z0 - 1) & 1][v * FNP + pidx(ex, ey)] = q[v];
     }
   }
 #pragma unroll
   for (int v = 0; v < 9; ++v) {
     Lzp[v] = T(0);
     Fzp[v] = T(0);
-    if (owned) dxy(v) = T(0);
+    if (owned && v < ND) dxy(v) = T(0);
   }
   T smax = T(0);
 
@@ -354,7 +369,7 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
     if (m - 1 >= z0 && stores) {
       T o[9];
       const int64_t idx = (int64_t)(m - 1) * g.plane + col;
-      load_cons<NARROW>(U, idx, o);
+      load_cons<NARROW, ND>(U, idx, o);
       if constexpr (CT) {
         ct_flush_cell(m);
         flushed = true;
@@ -365,12 +380,12 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
 #pragma unroll
         for (int v = 0; v < 9; ++v) {
           U0[v] = o[v];
-          du[v] = P.dtdx * (dxy(v) + (Fzp[v] - Fz[v]));
+          du[v] = v < ND ? P.dtdx * (dxy(v) + (Fzp[v] - Fz[v])) : T(0);
         }
         src_update(U0, du, o, src, idx, P, CT);
       } else {
 #pragma unroll
-        for (int v = 0; v < 9; ++v) o[v] += P.dtdx * (dxy(v) + (Fzp[v] - Fz[v]));
+        for (int v = 0; v < ND; ++v) o[v] += P.dtdx * (dxy(v) + (Fzp[v] - Fz[v]));
       }
       if constexpr (CT) {
         o[8] = T(0);  // no cleaning field under CT (integrator_ref.jl:150-158)
@@ -378,7 +393,8 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
         o[8] *= P.decay;
       }
 #pragma unroll
-      for (int v = 0; v < 9; ++v) *cell_at<NARROW>(O.v[v], idx) = o[v];
+      for (int v = 0; v < 9; ++v)
+        if (!CT || v < 5 || v == 8) *cell_at<NARROW>(O.v[v], idx) = o[v];
       // CT: the cell field is replaced by the face average after the step, so the CFL
       // speed is taken from the final state instead
       if constexpr (!CT) smax = nanmax(smax, cell_wavespeed(o, P));
@@ -388,7 +404,7 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
     }
     if (!first) {
 #pragma unroll
-      for (int v = 0; v < 9; ++v) Fzp[v] = Fz[v];
+      for (int v = 0; v < ND; ++v) Fzp[v] = Fz[v];
     }
 #pragma unroll
     for (int v = 0; v < 9; ++v) Lzp[v] = Lzn[v];
@@ -456,7 +472,7 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
       T q[9];
       cons2prim(Xc, q, P);
 #pragma unroll
-      for (int v = 0; v < 9; ++v) nxt[v * FNP + pidx(ex, ey)] = q[v];
+      for (int v = 0; v < NV; ++v) nxt[v * FNP + pidx(ex, ey)] = q[v];
     }
     if (has_col) {
       T q[9];
@@ -467,15 +483,15 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
     // (2) Hancock prediction of plane m (glm_physics.jl:225-231, integrator_ref.jl:17-26)
     T Rx[9], Ry[9], Rz[9], Lzn[9];
     if (stores || (pred_live && ring_work) || ezf || (ecorner && ring_work)) {
-      T m0[9], dLx[9], dRx[9], dLy[9], dRy[9], dLz[9], dRz[9];
+      T m0[9] = {}, dLx[9] = {}, dRx[9] = {}, dLy[9] = {}, dRy[9] = {}, dLz[9] = {}, dRz[9] = {};
       if constexpr (ZCARRY) {
         if (first) {
 #pragma unroll
-          for (int v = 0; v < 9; ++v) dzc[v] = cur[v * FNP + me] - nxt[v * FNP + me];
+          for (int v = 0; v < NV; ++v) dzc[v] = cur[v * FNP + me] - nxt[v * FNP + me];
         }
       }
 #pragma unroll
-      for (int v = 0; v < 9; ++v) {
+      for (int v = 0; v < NV; ++v) {
         m0[v] = cur[v * FNP + me];
         offsets<RECON>(cur[v * FNP + me - 1], m0[v], cur[v * FNP + me + 1], dLx[v], dRx[v]);
         offsets<RECON>(cur[v * FNP + me - FPW], m0[v], cur[v * FNP + me + FPW], dLy[v], dRy[v]);
@@ -573,20 +589,24 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
         }
         if (xleft) {
 #pragma unroll
-          for (int v = 0; v < 9; ++v) S.sLX[v * NFX + xl(ix, iy)] = fx[v];
+          for (int v = 0; v < 9; ++v)
+            if (xstate(v)) S.sLX[v * NFX + xl(ix, iy)] = fx[v];
         }
         if (yleft) {
 #pragma unroll
-          for (int v = 0; v < 9; ++v) S.sLY[v * NFY + yl(ix, iy)] = fy[v];
+          for (int v = 0; v < 9; ++v)
+            if (ystate(v)) S.sLY[v * NFY + yl(ix, iy)] = fy[v];
         }
       } else {
         if (xleft_e) {
 #pragma unroll
-          for (int v = 0; v < 9; ++v) S.sLX[v * NFX + xl(ix, iy)] = mh[v] + dRx[v];
+          for (int v = 0; v < 9; ++v)
+            if (xstate(v)) S.sLX[v * NFX + xl(ix, iy)] = mh[v] + dRx[v];
         }
         if (yleft_e) {
 #pragma unroll
-          for (int v = 0; v < 9; ++v) S.sLY[v * NFY + yl(ix, iy)] = mh[v] + dRy[v];
+          for (int v = 0; v < 9; ++v)
+            if (ystate(v)) S.sLY[v * NFY + yl(ix, iy)] = mh[v] + dRy[v];
         }
 #pragma unroll
         for (int v = 0; v < 9; ++v) {
@@ -678,7 +698,7 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
       // ring column with no prediction on this plane: still deposit plane m+1 (and carry
       // the column's z difference)
 #pragma unroll
-      for (int v = 0; v < 9; ++v) {
+      for (int v = 0; v < NV; ++v) {
         if constexpr (ZCARRY) dzc[v] = Pn[v] - cur[v * FNP + me];
         nxt[v * FNP + me] = Pn[v];
       }
@@ -764,7 +784,7 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
       if (xs) {
         T L[9];
 #pragma unroll
-        for (int v = 0; v < 9; ++v) L[v] = S.sLX[v * NFX + xl(ix - 1, iy)];
+        for (int v = 0; v < 9; ++v) L[v] = xstate(v) ? S.sLX[v * NFX + xl(ix - 1, iy)] : T(0);
         if constexpr (CT) {
           L[5] = bfx;
           Rx[5] = bfx;
@@ -780,12 +800,13 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
           face_flux<0, false, T, RS>(L, Rx, Fx, P);
         }
 #pragma unroll
-        for (int v = 0; v < 9; ++v) S.sLX[v * NFX + xl(ix - 1, iy)] = Fx[v];
+        for (int v = 0; v < 9; ++v)
+          if (xflux(v)) S.sLX[v * NFX + xl(ix - 1, iy)] = Fx[v];
       }
       if (ys) {
         T L[9];
 #pragma unroll
-        for (int v = 0; v < 9; ++v) L[v] = S.sLY[v * NFY + yl(ix, iy - 1)];
+        for (int v = 0; v < 9; ++v) L[v] = ystate(v) ? S.sLY[v * NFY + yl(ix, iy - 1)] : T(0);
         if constexpr (CT) {
           L[6] = bfy;
           Ry[6] = bfy;
@@ -801,13 +822,14 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
           face_flux<1, false, T, RS>(L, Ry, Fy, P);
         }
 #pragma unroll
-        for (int v = 0; v < 9; ++v) S.sLY[v * NFY + yl(ix, iy - 1)] = Fy[v];
+        for (int v = 0; v < 9; ++v)
+          if (yflux(v)) S.sLY[v * NFY + yl(ix, iy - 1)] = Fy[v];
       }
       }
       __syncthreads();
       if (stores) {
 #pragma unroll
-        for (int v = 0; v < 9; ++v)
+        for (int v = 0; v < ND; ++v)
           dxy(v) = (S.sLX[v * NFX + xl(ix - 1, iy)] - S.sLX[v * NFX + xl(ix, iy)]) +
                    (S.sLY[v * NFY + yl(ix, iy - 1)] - S.sLY[v * NFY + yl(ix, iy)]);
       }
@@ -1423,7 +1445,7 @@ template <class T, int RECON, int RS, bool SRC = false, bool NARROW = false, boo
 __device__ __forceinline__ void step_fused_ct_body(const Fields<const T>& U, const Fields<T>& O, T* __restrict__ ctp,
                                                    const FusedGeom& g, const StepParams<T>& P,
                                                    const SrcParams<T>& src = SrcParams<T>{}) {
-  __shared__ FusedLds<T, SRC, dxy_in_lds<RECON, false>(), EDGES> lds;
+  __shared__ FusedLds<T, SRC, dxy_in_lds<RECON, false>(), EDGES, true> lds;
   const int w = xcd_tile();
   unsigned none = 0;
   (void)fused_item<T, RECON, RS, false, SRC, NARROW, true, false, EDGES>(U, O, g, P, w, lds, nullptr, 0.f,
@@ -1453,11 +1475,13 @@ __global__ __launch_bounds__(FTHREADS) __attribute__((amdgpu_waves_per_eu(3))) v
   step_fused_ct_body<float, RECON, RS, false, NARROW, EDGES>(U, O, ctp, g, P);
 }
 
-// The in-step edge EMFs: float, three waves, no sources, and PLM (PPM's LDS divergence
-// carry leaves no room for the exchange arrays at three workgroups per CU).
+// The in-step edge EMFs: float, three waves and no sources. Without psi, the normal fields
+// and the updates of cell B the exchange arrays fit three workgroups a CU beside PPM's
+// divergence carry too (46.5 KB; 53.9 before): 96^3 PPM loop step 91 -> 59 us, 256^3 PPM 1.56 ms
+// with the slots, 1.27 with the edges; 256^3 minmod loop step 1265 -> 1131.
 template <int RECON, int RS>
 constexpr bool ct_edges_in_step() {
-  return RECON != RECON_PPM && ct_three_waves<RECON, RS>();
+  return ct_three_waves<RECON, RS>();
 }
 
 // The CT step with the drag / radiation sources (step_ref_drag! / step_ref_radiation! on

@@ -985,18 +985,12 @@ void launch_fused_variant(dim3 grd, hipStream_t st, const Fields<const T>& U, co
                        Pd, red, simg, thr, nsmooth, src);
 }
 
-// The plain float step with 32-bit offsets (double steps never take this path).
-template <class T, int RECON, int RS>
-void launch_plain_narrow(dim3 grd, hipStream_t st, const Fields<const T>& U, const Fields<T>& O, const FusedGeom& g,
-                         const StepParams<T>& P, double* red, const StepParams<T>* Pd) {
-  if constexpr (sizeof(T) == 4)
-    launch_fused_variant<T, RECON, RS, false, false, true>(grd, st, U, O, g, P, red, nullptr, 0.f, nullptr,
-                                                           SrcParams<T>{}, Pd);
-}
-
-// Fields of nc cells addressable with 32-bit byte offsets. PMFMHD_WIDE_OFFSETS=1 in the
-// environment selects the 64-bit-offset kernels for every grid (they otherwise run only
-// for float fields of 4 GiB and more, 1024^3 and up), so that tests can compare the two.
+// Fields of nc cells addressable with 32-bit byte offsets: each access is then a scalar base
+// plus one VGPR, without the 64-bit address pairs (of the step's VALU instructions 2 to 3%:
+// 2560 -> 2490 plain, 3428 -> 3369 drag, 2763 -> 2690 with boundaries, 3409 -> 3337 with the
+// surrogate, 3635 -> 3566 float64). PMFMHD_WIDE_OFFSETS=1 in the environment selects the
+// 64-bit-offset kernels for every grid (they otherwise run only for fields of 4 GiB and more,
+// 1024^3 float32 and 813^3 float64 up), so that tests can compare the two.
 template <class T> inline bool narrow_fields(int64_t nc) {
   const char* wide = std::getenv("PMFMHD_WIDE_OFFSETS");
   if (wide && wide[0] == '1') return false;
@@ -1198,16 +1192,20 @@ bool launch_step_fused(Fields<const T> U, Fields<T> O, const Grid& G, const Step
   FusedGeom g = fused_geom(G, chunk_of(G, zc, sizeof(T) == 8));
   unsigned nb = (unsigned)((int64_t)g.ntx * g.nty * g.nchunks);
   dim3 blk(FTHREADS), grd(nb);
-  const bool narrow = sizeof(T) == 4 && narrow_fields<T>(G.nc);
+  const bool narrow = narrow_fields<T>(G.nc);
   const bool gen = !all_periodic(G);  // outflow / reflecting axes: the BCG variants
-#define PMF_FUSED(R, S)                                                                                             \
-  if (gen && src)                                                                                                  \
-    launch_fused_variant<T, R, S, false, true, false, true>(grd, st, U, O, g, P, red, nullptr, 0.f, nullptr, *src); \
-  else if (gen) launch_fused_variant<T, R, S, false, false, false, true>(grd, st, U, O, g, P, red, nullptr, 0.f,     \
-                                                                         nullptr, SrcParams<T>{}, Pd);              \
-  else if (src) launch_fused_variant<T, R, S, false, true>(grd, st, U, O, g, P, red, nullptr, 0.f, nullptr, *src);   \
-  else if (narrow) launch_plain_narrow<T, R, S>(grd, st, U, O, g, P, red, Pd);                                      \
-  else launch_fused_variant<T, R, S, false, false>(grd, st, U, O, g, P, red, nullptr, 0.f, nullptr, SrcParams<T>{}, Pd)
+#define PMF_FUSED_V(R, S, SRC, BCG)                                                                             \
+  do {                                                                                                          \
+    const SrcParams<T> sp = SRC ? *src : SrcParams<T>{};                                                        \
+    const StepParams<T>* pd = SRC ? nullptr : Pd;                                                               \
+    if (narrow) launch_fused_variant<T, R, S, false, SRC, true, BCG>(grd, st, U, O, g, P, red, nullptr, 0.f, nullptr, sp, pd); \
+    else launch_fused_variant<T, R, S, false, SRC, false, BCG>(grd, st, U, O, g, P, red, nullptr, 0.f, nullptr, sp, pd); \
+  } while (0)
+#define PMF_FUSED(R, S)                           \
+  if (gen && src) PMF_FUSED_V(R, S, true, true);  \
+  else if (gen) PMF_FUSED_V(R, S, false, true);   \
+  else if (src) PMF_FUSED_V(R, S, true, false);   \
+  else PMF_FUSED_V(R, S, false, false)
 #define PMF_FUSED_RS(R)                                  \
   if (P.rsolve == RS_HLL) PMF_FUSED(R, RS_HLL);          \
   else if (P.rsolve == RS_LLF) PMF_FUSED(R, RS_LLF);     \
@@ -1221,6 +1219,7 @@ bool launch_step_fused(Fields<const T> U, Fields<T> O, const Grid& G, const Step
   }
 #undef PMF_FUSED_RS
 #undef PMF_FUSED
+#undef PMF_FUSED_V
   if (dsmax) launch_fold_max(red, nb, dsmax, hsmax, st);
   return true;
 }
@@ -1230,9 +1229,14 @@ bool launch_step_fused_surr(Fields<const float> U, Fields<float> O, const Grid& 
                             unsigned long long* nsmooth, hipStream_t st, double* hsmax) {
   if (!surrogate_grid(G) || P.rsolve != RS_HLLD) return false;
   FusedGeom g = fused_geom(G, pick_zc(G, 2));
+  const bool narrow = narrow_fields<float>(G.nc);
   unsigned nb = (unsigned)((int64_t)g.ntx * g.nty * g.nchunks);
   dim3 blk(FTHREADS), grd(nb);
-#define PMF_FUSED_S(R) launch_fused_variant<float, R, RS_HLLD, true>(grd, st, U, O, g, P, red, simg, thr, nsmooth)
+#define PMF_FUSED_S(R)                                                                                          \
+  do {                                                                                                          \
+    if (narrow) launch_fused_variant<float, R, RS_HLLD, true, false, true>(grd, st, U, O, g, P, red, simg, thr, nsmooth); \
+    else launch_fused_variant<float, R, RS_HLLD, true, false, false>(grd, st, U, O, g, P, red, simg, thr, nsmooth); \
+  } while (0)
   if (P.recon == RECON_PPM) PMF_FUSED_S(RECON_PPM);
   else if (P.recon == RECON_PLM_MINMOD) PMF_FUSED_S(RECON_PLM_MINMOD);
   else PMF_FUSED_S(RECON_PLM);

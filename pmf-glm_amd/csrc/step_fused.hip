@@ -196,7 +196,7 @@ template <class T> __device__ __forceinline__ void cell_emf(const T* v, const T*
 // GS05 upwind average) from the face fluxes and cell EMFs it has just computed, and writes
 // them to workspace slots 15-17 instead of writing slots 3-14 for a separate edge pass.
 template <class T, int RECON, int RS, bool SURR, bool SRC = false, bool NARROW = false, bool CT = false,
-          bool BCG = false, bool EDGES = false>
+          bool BCG = false, bool EDGES = false, bool AHEAD = false>
 __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T>& O, const FusedGeom& g,
                                         const StepParams<T>& P, int w,
                                         FusedLds<T, SRC, dxy_in_lds<RECON, SURR>(), EDGES, CT>& S,
@@ -417,6 +417,28 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
   // it)
   constexpr bool ZCARRY = RECON != RECON_PPM && !SRC && !SURR && sizeof(T) == 4;
   T dzc[9];
+  // The loads of plane m's pass: plane m+1 of the own column and of the extra cell; SRC: the
+  // radiation correction and the fallback mask of plane m's predicted cell (used after the
+  // prediction). Issued at the pass's start, or (AHEAD) before the x and y faces of plane m-1.
+  struct Loads {
+    T own[9], extra[9], cv[3], mkv;
+    __device__ __forceinline__ Loads() { cv[0] = cv[1] = cv[2] = mkv = T(0); }
+  };
+  auto fetch = [&](int m, Loads& f) {
+    if (has_col) load_plane(m + 1, col, 0, f.own);
+    if (has_extra && m + 1 < z0 + zc) load_plane(m + 1, ecol, 2, f.extra);
+    if constexpr (SRC) {
+      if (has_col) {
+        const int64_t pc = (int64_t)wrapi(m, g.nz) * g.plane + pcol;
+        if (src.flags & SRC_RAD) {
+#pragma unroll
+          for (int c = 0; c < 3; ++c) f.cv[c] = src.corr[(1 + c) * src.stride + pc];
+        }
+        if (src.check == CHECK_MASKED) f.mkv = src.corr[4 * src.stride + pc];
+      }
+    }
+  };
+  Loads ahead;
   for (int m = z0 - 1; m <= z0 + zc; ++m) {
     const bool first = m == z0 - 1, last = m == z0 + zc;
     const bool ring_work = !(first || last);  // ring columns feed x/y faces only
@@ -428,24 +450,13 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
     const T* __restrict__ cur = S.sP[m & 1];
     T* __restrict__ nxt = S.sP[(m + 1) & 1];   // holds plane m-1 now, plane m+1 after this pass
     // (1) plane m+1 of the own column and of the extra cell (in flight during the barrier)
-    T Pn[9], Xc[9];
-    if (has_col) load_plane(m + 1, col, 0, Pn);
+    Loads now;
+    Loads& f = AHEAD ? ahead : now;
+    if (!AHEAD || first) fetch(m, f);
+    T* const Pn = f.own;
+    const T *Xc = f.extra, *cv = f.cv;
+    const T mkv = f.mkv;
     const bool extra_now = has_extra && m + 1 < z0 + zc;
-    if (extra_now) load_plane(m + 1, ecol, 2, Xc);
-    // SRC: the radiation correction and the fallback mask of this plane's predicted cell,
-    // also in flight during the barrier (they are used after the prediction)
-    T cv[3] = {T(0), T(0), T(0)};
-    T mkv = T(0);
-    if constexpr (SRC) {
-      if (has_col) {
-        const int64_t pc = (int64_t)wrapi(m, g.nz) * g.plane + pcol;
-        if (src.flags & SRC_RAD) {
-#pragma unroll
-          for (int c = 0; c < 3; ++c) cv[c] = src.corr[(1 + c) * src.stride + pc];
-        }
-        if (src.check == CHECK_MASKED) mkv = src.corr[4 * src.stride + pc];
-      }
-    }
     // CT: the face fields this thread's solves take as the normal field (the z face m-1/2
     // of an owned column, the x and y faces of plane m), also in flight during the barrier
     T bfz = T(0), bfx = T(0), bfy = T(0);
@@ -704,6 +715,9 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
       }
     }
     __syncthreads();
+    if constexpr (AHEAD) {
+      if (!last) fetch(m + 1, ahead);
+    }
     // (3b) x and y faces of plane m, each solved once
     const bool xy = EDGES ? !last : !(first || last);
     if constexpr (SURR) {
@@ -907,7 +921,7 @@ constexpr bool fused_two_waves() {
 
 // The single-grid step: one workgroup per work item. simg is the network's image in
 // global memory (SURR only) and nsmooth the count of network-solved faces.
-template <class T, int RECON, int RS, bool SURR, bool SRC, bool NARROW, bool BCG = false>
+template <class T, int RECON, int RS, bool SURR, bool SRC, bool NARROW, bool BCG, bool AHEAD = false>
 __device__ __forceinline__ void step_fused_body(const Fields<const T>& U, const Fields<T>& O, const FusedGeom& g,
                                                 const StepParams<T>& P, double* __restrict__ red,
                                                 const unsigned char* __restrict__ simg, float thr,
@@ -926,7 +940,8 @@ __device__ __forceinline__ void step_fused_body(const Fields<const T>& U, const 
   SurrQueue<FQCAP>* q = nullptr;
   if constexpr (SURR) q = &sQ;
   const T smax =
-      fused_item<T, RECON, RS, SURR, SRC, NARROW, false, BCG>(U, O, g, P, w, lds, sW, thr, smooth_count, src, q);
+      fused_item<T, RECON, RS, SURR, SRC, NARROW, false, BCG, false, AHEAD>(U, O, g, P, w, lds, sW, thr, smooth_count,
+                                                                           src, q);
   // fold the workgroup's CFL maximum (timestep.jl:8-12 on the new state)
   block_store_max(smax, sMax, red + blockIdx.x);
   if constexpr (SURR) {
@@ -948,13 +963,13 @@ __global__ __launch_bounds__(FTHREADS) void k_step_fused(Fields<const T> U, Fiel
   step_fused_body<T, RECON, RS, SURR, SRC, NARROW, BCG>(U, O, g, P, red, simg, thr, nsmooth, src);
 }
 
-template <class T, int RECON, int RS, bool SURR, bool SRC, bool NARROW, bool BCG>
+template <class T, int RECON, int RS, bool SURR, bool SRC, bool NARROW, bool BCG, bool AHEAD>
 __global__ __launch_bounds__(FTHREADS) __attribute__((amdgpu_waves_per_eu(3))) void k_step_fused3(
     Fields<const T> U, Fields<T> O, FusedGeom g, StepParams<T> P, const StepParams<T>* __restrict__ Pd,
     double* __restrict__ red, const unsigned char* __restrict__ simg, float thr,
     unsigned long long* __restrict__ nsmooth, SrcParams<T> src) {
   if (Pd) P = *Pd;
-  step_fused_body<T, RECON, RS, SURR, SRC, NARROW, BCG>(U, O, g, P, red, simg, thr, nsmooth, src);
+  step_fused_body<T, RECON, RS, SURR, SRC, NARROW, BCG, AHEAD>(U, O, g, P, red, simg, thr, nsmooth, src);
 }
 
 // Two waves per SIMD. The surrogate-assisted step: about 250 VGPRs with the network in its
@@ -969,15 +984,44 @@ __global__ __launch_bounds__(FTHREADS) __attribute__((amdgpu_waves_per_eu(2))) v
   step_fused_body<T, RECON, RS, SURR, SRC, NARROW, BCG>(U, O, g, P, red, simg, thr, nsmooth, src);
 }
 
+// Compute units of the current device (cached per device).
+static int device_cus() {
+  static int cus[64] = {0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (!cus[dev]) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    cus[dev] = n;
+  }
+  return cus[dev];
+}
+
+// Whether a periodic float step issues each pass's loads before the x and y faces of the pass
+// before (fused_item's AHEAD), which cover them, instead of at the pass's start, where only the
+// barrier and the CU's other workgroups do: 256^3 minmod 800 -> 770 us, 512^3 6520 -> 6210,
+// 128^3 PPM (704 workgroups) 104 -> 97.6, 160^3 minmod (700) 224 -> 212, 192^3 tracked
+// radiation 515 -> 488. Only where CUs hold a third workgroup: with one or two the step is a
+// chain of few waves, and the 18 values carried from pass to pass add to it (64^3 minmod, 384
+// workgroups: 27.4 us, 28.6 with; 32^3, 192: 14.4, 14.7). With boundaries it costs 4%; the
+// edge-forming CT steps and the ensemble gain nothing.
+static bool loads_ahead(unsigned groups) { return groups > 2u * (unsigned)device_cus(); }
+
 template <class T, int RECON, int RS, bool SURR, bool SRC = false, bool NARROW = false, bool BCG = false>
 void launch_fused_variant(dim3 grd, hipStream_t st, const Fields<const T>& U, const Fields<T>& O, const FusedGeom& g,
                           const StepParams<T>& P, double* red, const unsigned char* simg, float thr,
                           unsigned long long* nsmooth, const SrcParams<T>& src = SrcParams<T>{},
                           const StepParams<T>* Pd = nullptr) {
-  if constexpr (fused_three_waves<T, RECON, RS, SURR, SRC>())
-    hipLaunchKernelGGL((k_step_fused3<T, RECON, RS, SURR, SRC, NARROW, BCG>), grd, dim3(FTHREADS), 0, st, U, O, g, P,
-                       Pd, red, simg, thr, nsmooth, src);
-  else if constexpr (fused_two_waves<T, RECON, SURR, SRC>())
+  if constexpr (fused_three_waves<T, RECON, RS, SURR, SRC>()) {
+    bool ahead = !BCG;
+    if constexpr (NARROW) ahead = ahead && loads_ahead(grd.x);
+    if (ahead)
+      hipLaunchKernelGGL((k_step_fused3<T, RECON, RS, SURR, SRC, NARROW, BCG, !BCG>), grd, dim3(FTHREADS), 0, st, U, O,
+                         g, P, Pd, red, simg, thr, nsmooth, src);
+    else if constexpr (NARROW || BCG)
+      hipLaunchKernelGGL((k_step_fused3<T, RECON, RS, SURR, SRC, NARROW, BCG, false>), grd, dim3(FTHREADS), 0, st, U,
+                         O, g, P, Pd, red, simg, thr, nsmooth, src);
+  } else if constexpr (fused_two_waves<T, RECON, SURR, SRC>())
     hipLaunchKernelGGL((k_step_fused2<T, RECON, RS, SURR, SRC, NARROW, BCG>), grd, dim3(FTHREADS), 0, st, U, O, g, P,
                        Pd, red, simg, thr, nsmooth, src);
   else
@@ -1122,19 +1166,6 @@ bool all_periodic(const Grid& G) {
 
 // The surrogate step's grids: periodic, whole x tiles, ny and nz of at least two.
 bool surrogate_grid(const Grid& G) { return all_periodic(G) && G.nx % TX == 0 && G.ny >= 2 && G.nz >= 2; }
-
-// Compute units of the current device (cached per device).
-static int device_cus() {
-  static int cus[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (!cus[dev]) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cus[dev] = n;
-  }
-  return cus[dev];
-}
 
 // z-chunk length. A chunk of zc planes costs about zc + 2 of them (two more planes are
 // predicted at its ends), and a CU that holds 1, 2 or 3 workgroups steps a plane of each

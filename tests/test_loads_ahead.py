@@ -1,0 +1,43 @@
+"""The instances that load a pass ahead (more than two workgroups a CU) against the others: a
+state repeated along every axis steps to its own repetition, bit for bit, ragged tiles and a
+short last chunk included."""
+import numpy as np
+import pytest
+
+import pmfmhd as M
+from pmfmhd import problems as P
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dims", [(48, 48, 40), (50, 41, 42)])
+@pytest.mark.parametrize("recon,riemann", [("plm_minmod", "hlld"), ("plm", "hll"), ("ppm", "llf"), ("ppm", "hlld")])
+@pytest.mark.parametrize("kind", ["plain", "drag", "radiation"])
+def test_repeated_state_steps_to_its_repetition(dims, recon, riemann, kind):
+    nx, ny, nz = dims
+    n = nx * ny * nz
+    rng = np.random.default_rng(9)
+    one = np.ones(n)
+    q = [one + 0.2 * rng.uniform(-1, 1, n), *rng.normal(0, 0.3, (3, n)), one, *rng.normal(0, 0.4, (3, n)),
+         rng.normal(0, 0.05, n)]
+    U = P.prim2cons(q, 5.0 / 3.0).astype(np.float32).reshape(9, nz, ny, nx)
+    corr = np.zeros((9, nz, ny, nx))
+    corr[1:4] = 0.01 * rng.normal(size=(3, nz, ny, nx))
+    out = []
+    for r in (1, 2):  # at least 960 workgroups of four planes, and an eighth of them
+        s = M.allocate_state((r * nx, r * ny, r * nz), 0.1, dtype=np.float32, recon=recon, riemann=riemann)
+        s.set_conserved(np.tile(U, (1, r, r, r)).reshape(9, -1))
+        M.set_chunk(s, 4)
+        for _ in range(2):
+            if kind == "plain":
+                M.step(s, 2e-3, ch=3.0, integrator="cube")
+            elif kind == "drag":
+                M.step_drag(s, 2e-3, 3.0, 0.98, 0.2, integrator="cube")
+            else:
+                buf = M.correction_buffer(s, np.tile(corr, (1, r, r, r)).reshape(9, -1))
+                M.load_psi(s, buf)
+                M.step_radiation(s, 2e-3, 3.0, 0.98, 0.2, buf)
+        out.append((s.conserved().reshape(9, r * nz, r * ny, r * nx), M.max_wavespeed(s)))
+    assert np.all(np.isfinite(out[0][0]))
+    assert np.array_equal(np.tile(out[0][0], (1, 2, 2, 2)), out[1][0])
+    assert out[0][1] == out[1][1]

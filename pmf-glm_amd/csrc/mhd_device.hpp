@@ -479,11 +479,11 @@ __device__ __forceinline__ void hlld_guarded_n(const T* L, const T* R, T bn, T f
 // with that state's v, b and E, and equals F_side + S (U* - U_side) [+ S* (U** - U*)] of
 // hlld_guarded_n. So the outer states enter through E* only, U** is U* plus the Alfven jump
 // (db = sign(bn) sqrt(rho*) dv), pt* comes from the selected side, and the two fast speeds
-// share their outer root. The fused step is bound by VALU issue (0.96 of the peak rate): about
-// 220 issue slots per face instead of 275 took two 256^3 minmod steps from 1694 to 1610 us, a
-// 512^3 step from 6.80 to 6.56 ms, a 128^3 PPM step from 110 to 105 us. A face with a floored star
-// density or a degenerate star state (found from values this path needs anyway) goes to
-// hlld_guarded_n, in a branch that no wave of an ordinary flow takes. Pinned (explicit FMAs
+// share their outer root. The fused step is bound by VALU issue (active 0.99 of the CUs' busy
+// cycles): about 220 issue slots per face instead of 275 took two 256^3 minmod steps from 1694
+// to 1610 us, a 512^3 step from 6.80 to 6.56 ms, a 128^3 PPM step from 110 to 105 us. A face with
+// a floored star density or a degenerate star state (found from values this path needs anyway)
+// goes to hlld_guarded_n, in a branch that no wave of an ordinary flow takes. Pinned (explicit FMAs
 // only): every kernel that inlines it gives the same bits.
 template <class T>
 __device__ __forceinline__ void hlld_n(const T* L, const T* R, T bn, T fbn, T fpsi, T* f, const StepParams<T>& P,

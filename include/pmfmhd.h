@@ -165,9 +165,11 @@ int pmf_set_ct_kernel(pmf_state* s, int32_t per_cell);
 /* Workspace slots of the fused CT step. The reference's step writes every face's mass and
  * transverse-field fluxes and every cell's EMF to slots 3-14 of the CTState buffer, and
  * ct_update! forms the edge EMFs (slots 15-17) from them (integrator_ref.jl:83-139,
- * ct.jl:71-93). By default (fill = 0) the fused float step forms the edge EMFs
- * itself, bit for bit as that pass would, and leaves slots 3-14 as they were: every
- * reader of those slots in the reference writes them first. fill != 0 writes slots 3-14
+ * ct.jl:71-93). By default the fused float step (but for minmod with LLF, which always
+ * writes the slots and runs that pass, as float64 and source steps do) forms the edge EMFs
+ * itself, bit for bit as that pass would; with PLM or MonCen it leaves slots 3-14 as they
+ * were (every reader of those slots in the reference writes them first), with PPM it writes
+ * them too. fill = 0 leaves them as they were with PPM as well. fill != 0 writes slots 3-14
  * and runs the separate edge pass, as the reference does. No counterpart in the reference
  * (its step always writes them); cells, faces, edge EMFs and remainders are the same
  * either way. */

@@ -92,7 +92,7 @@ bool step_fields(pmf_state* s, Fields<const T> in, Fields<T> out, T* ctp, double
     // variant allows, the edge EMFs of ct_update! come out of the same kernel
     mark(s);
     launch_step_fused_ct<T>(in, out, ctp, s->G, make_params<T>(s, dt, 0.0, 1.0), s->st, s->zc, nullptr,
-                            !s->ct_fill_workspace, &edges);
+                            s->ct_workspace, &edges);
     mark(s);
   } else {
     mark(s);
@@ -467,7 +467,7 @@ int pmf_set_ct_kernel(pmf_state* s, int32_t per_cell) {
 int pmf_set_ct_workspace(pmf_state* s, int32_t fill) {
   return guard([&] {
     check_state(s);
-    s->ct_fill_workspace = fill != 0;
+    s->ct_workspace = fill != 0 ? CT_FILL : CT_LEAVE;
   });
 }
 
@@ -629,11 +629,11 @@ int pmf_autotune(pmf_state* s, int32_t reps, int32_t* zc_out, double* ms_out) {
           if (ct && s->p.precision == PMF_F64)
             launch_step_fused_ct<double>(cfields_at<double>(s->U, s->nc), fields_at<double>(s->S, s->nc),
                                          (double*)s->ct, s->G, make_params<double>(s, dt, 0.0, 1.0), s->st, s->zc,
-                                         nullptr, !s->ct_fill_workspace);
+                                         nullptr, s->ct_workspace);
           else if (ct)
             launch_step_fused_ct<float>(cfields_at<float>(s->U, s->nc), fields_at<float>(s->S, s->nc),
                                         (float*)s->ct, s->G, make_params<float>(s, dt, 0.0, 1.0), s->st, s->zc,
-                                        nullptr, !s->ct_fill_workspace);
+                                        nullptr, s->ct_workspace);
           else if (s->p.precision == PMF_F64)
             step_fields<double>(s, cfields_at<double>(s->U, s->nc), fields_at<double>(s->S, s->nc), nullptr, dt, ch,
                                 1.0, PMF_INTEGRATOR_CUBE, true);

@@ -45,13 +45,14 @@ bool surrogate_grid(const Grid& G);
 // The fused CT step (constrained-transport states, the :ref algorithm with each face
 // solved once): the cell update into O and workspace slots 3-14 of ctp; ct_update! then
 // finishes the step. src: the drag / radiation sources (no fallback masks: those belong
-// to the :cube integrator). want_edges: where the variant supports it, form the edge
-// EMFs (slots 15-17) in the step instead of writing slots 3-14; *edges tells whether it
-// did (then ct_update! skips its edge pass). Returns false when the grid shape is not
-// supported.
+// to the :cube integrator). Unless workspace is CT_FILL, a variant that supports it forms the
+// edge EMFs (slots 15-17) in the step, and writes slots 3-14 only with PPM under CT_DEFAULT;
+// *edges tells whether it did (then ct_update! skips its edge pass). Returns false when the grid
+// shape is not supported.
+enum { CT_DEFAULT = -1, CT_LEAVE = 0, CT_FILL = 1 };  // workspace slots 3-14: not said, not needed, needed
 template <class T>
 bool launch_step_fused_ct(Fields<const T> U, Fields<T> O, T* ctp, const Grid& G, const StepParams<T>& P,
-                          hipStream_t st, int zc = 0, const SrcParams<T>* src = nullptr, bool want_edges = false,
+                          hipStream_t st, int zc = 0, const SrcParams<T>* src = nullptr, int workspace = CT_FILL,
                           bool* edges = nullptr);
 // The surrogate-assisted fused step (float32, HLLD): simg is the network's LDS image,
 // nsmooth accumulates the number of faces solved by the network.

@@ -55,10 +55,11 @@ struct pmf_state {
   bool smax_valid = false;  // dval[0] holds the CFL speed of the current U
   int zc = 0;               // planes per z chunk of the fused kernel (0 = built-in choice)
   bool percell = false;  // :ref steps on the per-cell kernel even where the fused one applies
-  // CT steps on the fused kernel also write workspace slots 3-14 (face mass and field fluxes,
-  // cell EMFs) and form the edge EMFs in a separate pass, as the reference's step does;
-  // otherwise the fused kernel forms the edge EMFs itself and leaves slots 3-14 alone
-  bool ct_fill_workspace = false;
+  // CT steps on the fused kernel: CT_FILL writes workspace slots 3-14 (face mass and field
+  // fluxes, cell EMFs) and forms the edge EMFs in a separate pass, as the reference's step does;
+  // otherwise the kernel forms the edge EMFs itself and leaves slots 3-14 alone (CT_DEFAULT: but
+  // for PPM steps)
+  int ct_workspace = pmf::CT_DEFAULT;
   bool timing = false;      // bracket step kernels with events
   std::vector<hipEvent_t> ev;  // pairs (start, stop) in launch order
   size_t ev_used = 0;

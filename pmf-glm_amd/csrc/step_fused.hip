@@ -194,9 +194,10 @@ template <class T> __device__ __forceinline__ void cell_emf(const T* v, const T*
 
 // EDGES (CT only): the step also forms the edge EMFs of its stored cells (ct.jl:71-93, the
 // GS05 upwind average) from the face fluxes and cell EMFs it has just computed, and writes
-// them to workspace slots 15-17 instead of writing slots 3-14 for a separate edge pass.
+// them to workspace slots 15-17 instead of writing slots 3-14 for a separate edge pass. FILL:
+// slots 3-14 are written as well, from the LDS copies that the edges are formed from.
 template <class T, int RECON, int RS, bool SURR, bool SRC = false, bool NARROW = false, bool CT = false,
-          bool BCG = false, bool EDGES = false, bool AHEAD = false>
+          bool BCG = false, bool EDGES = false, bool AHEAD = false, bool FILL = false>
 __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T>& O, const FusedGeom& g,
                                         const StepParams<T>& P, int w,
                                         FusedLds<T, SRC, dxy_in_lds<RECON, SURR>(), EDGES, CT>& S,
@@ -205,6 +206,7 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
   static_assert(!(CT && SURR), "the fused CT step has no surrogate");
   static_assert(!(BCG && (CT || SURR)), "the CT and surrogate steps run on periodic grids");
   static_assert(!EDGES || (CT && !SRC), "edge EMFs belong to the plain CT step");
+  static_assert(!FILL || EDGES, "without the edges the CT step always writes slots 3-14");
   // Under CT psi takes no part (its flux is zero and the step clears it), the normal field of a
   // face state is the face field, and cell B is the face average after the step, so its
   // update is left out unless the sources' energy floor reads it. NV: fields that are loaded
@@ -473,6 +475,24 @@ __device__ __forceinline__ T fused_item(const Fields<const T>& U, const Fields<T
         ctslot(4, idx) = ctxy[3];
         ctslot(8, idx) = ctxy[4];
         ctslot(9, idx) = ctxy[5];
+      }
+      // FILL: plane m-1's fluxes and cell EMFs, which its edges were formed from, still in LDS
+      if (FILL && stores && m - 1 >= z0) {
+        const int64_t idx = (int64_t)(m - 1) * g.plane + col;
+        const int q = qidx(ix, iy), xo = xl(ix - 1, iy), yo = yl(ix, iy - 1);
+        const T* E = S.sExy + ((m - 1) & 1) * 2 * FNQ;
+        ctslot(3, idx) = S.sLX[xo];
+        ctslot(4, idx) = S.sLY[yo];
+        ctslot(5, idx) = S.sZf[q];
+        ctslot(6, idx) = S.sLX[6 * NFX + xo];
+        ctslot(7, idx) = S.sLX[7 * NFX + xo];
+        ctslot(8, idx) = S.sLY[5 * NFY + yo];
+        ctslot(9, idx) = S.sLY[7 * NFY + yo];
+        ctslot(10, idx) = S.sZf[FNQ + q];
+        ctslot(11, idx) = S.sZf[2 * FNQ + q];
+        ctslot(12, idx) = E[q];
+        ctslot(13, idx) = E[FNQ + q];
+        ctslot(14, idx) = S.sEz[q];
       }
     }
     if constexpr (SURR) {
@@ -1476,15 +1496,15 @@ void launch_ens_step(const EnsCube* cubes, const int2* items, const EnsQueues& q
 // the face fields, integrator_ref.jl:83-139) with each face solved once; writes the cell
 // update and workspace slots 3-14 (face mass and transverse-B fluxes of every cell's
 // lower faces, cell EMFs) that ct_update! reads.
-template <class T, int RECON, int RS, bool SRC = false, bool NARROW = false, bool EDGES = false>
+template <class T, int RECON, int RS, bool SRC = false, bool NARROW = false, bool EDGES = false, bool FILL = false>
 __device__ __forceinline__ void step_fused_ct_body(const Fields<const T>& U, const Fields<T>& O, T* __restrict__ ctp,
                                                    const FusedGeom& g, const StepParams<T>& P,
                                                    const SrcParams<T>& src = SrcParams<T>{}) {
   __shared__ FusedLds<T, SRC, dxy_in_lds<RECON, false>(), EDGES, true> lds;
   const int w = xcd_tile();
   unsigned none = 0;
-  (void)fused_item<T, RECON, RS, false, SRC, NARROW, true, false, EDGES>(U, O, g, P, w, lds, nullptr, 0.f,
-                                                                         none, src, nullptr, ctp);
+  (void)fused_item<T, RECON, RS, false, SRC, NARROW, true, false, EDGES, false, FILL>(U, O, g, P, w, lds, nullptr, 0.f,
+                                                                                      none, src, nullptr, ctp);
 }
 
 template <class T, int RECON, int RS>
@@ -1503,20 +1523,27 @@ constexpr bool ct_three_waves() {
 
 // NARROW: every field and every slot of the packed buffer is addressed as its scalar base
 // plus a 32-bit byte offset (fields below 4 GiB). EDGES: the step forms the edge EMFs
-// (slots 15-17) itself and leaves slots 3-14 alone.
-template <int RECON, int RS, bool NARROW, bool EDGES = false>
+// (slots 15-17) itself and leaves slots 3-14 alone, or (FILL) writes them too.
+template <int RECON, int RS, bool NARROW, bool EDGES = false, bool FILL = false>
 __global__ __launch_bounds__(FTHREADS) __attribute__((amdgpu_waves_per_eu(3))) void k_step_fused_ct3(
     Fields<const float> U, Fields<float> O, float* __restrict__ ctp, FusedGeom g, StepParams<float> P) {
-  step_fused_ct_body<float, RECON, RS, false, NARROW, EDGES>(U, O, ctp, g, P);
+  step_fused_ct_body<float, RECON, RS, false, NARROW, EDGES, FILL>(U, O, ctp, g, P);
 }
 
 // The in-step edge EMFs: float, three waves and no sources. Without psi, the normal fields
 // and the updates of cell B the exchange arrays fit three workgroups a CU beside PPM's
-// divergence carry too (46.5 KB; 53.9 before): 96^3 PPM loop step 91 -> 59 us, 256^3 PPM 1.56 ms
-// with the slots, 1.27 with the edges; 256^3 minmod loop step 1265 -> 1131.
+// divergence carry too (46.5 KB; 53.9 before): 96^3 PPM loop step 91 -> 59 us (70.5 with slots
+// 3-14 written as well, 42 MB), 256^3 minmod loop step 1265 -> 1131.
 template <int RECON, int RS>
 constexpr bool ct_edges_in_step() {
   return ct_three_waves<RECON, RS>();
+}
+
+// Whether the step that forms its edges also writes slots 3-14 unless the caller has said that
+// it does not read them (CT_LEAVE): a PPM step always has.
+template <int RECON>
+constexpr bool ct_edge_step_fills() {
+  return RECON == RECON_PPM;
 }
 
 // The CT step with the drag / radiation sources (step_ref_drag! / step_ref_radiation! on
@@ -1530,7 +1557,7 @@ __global__ __launch_bounds__(FTHREADS) void k_step_fused_ct_src(Fields<const T> 
 
 template <class T>
 bool launch_step_fused_ct(Fields<const T> U, Fields<T> O, T* ctp, const Grid& G, const StepParams<T>& P,
-                          hipStream_t st, int zc, const SrcParams<T>* src, bool want_edges, bool* edges) {
+                          hipStream_t st, int zc, const SrcParams<T>* src, int workspace, bool* edges) {
   if (edges) *edges = false;
   if (!fused_supported(G, sizeof(T) == 8, P.recon, P.rsolve) || !all_periodic(G)) return false;
   FusedGeom g = fused_geom(G, chunk_of(G, zc, sizeof(T) == 8));
@@ -1542,8 +1569,14 @@ bool launch_step_fused_ct(Fields<const T> U, Fields<T> O, T* ctp, const Grid& G,
       hipLaunchKernelGGL((k_step_fused_ct_src<T, R, S>), grd, blk, 0, st, U, O, ctp, g, P, *src); \
     else if constexpr (sizeof(T) == 4 && ct_three_waves<R, S>()) {                    \
       if constexpr (ct_edges_in_step<R, S>()) {                                        \
-        if (want_edges) {                                                              \
-          if (narrow)                                                                  \
+        constexpr bool kFill = ct_edge_step_fills<R>();                                \
+        if (workspace != CT_FILL) {                                                    \
+          const bool fill = kFill && workspace == CT_DEFAULT;                          \
+          if (narrow && fill)                                                          \
+            hipLaunchKernelGGL((k_step_fused_ct3<R, S, true, true, kFill>), grd, blk, 0, st, U, O, ctp, g, P); \
+          else if (fill)                                                               \
+            hipLaunchKernelGGL((k_step_fused_ct3<R, S, false, true, kFill>), grd, blk, 0, st, U, O, ctp, g, P); \
+          else if (narrow)                                                             \
             hipLaunchKernelGGL((k_step_fused_ct3<R, S, true, true>), grd, blk, 0, st, U, O, ctp, g, P); \
           else                                                                         \
             hipLaunchKernelGGL((k_step_fused_ct3<R, S, false, true>), grd, blk, 0, st, U, O, ctp, g, P); \
@@ -1575,10 +1608,10 @@ bool launch_step_fused_ct(Fields<const T> U, Fields<T> O, T* ctp, const Grid& G,
 }
 
 template bool launch_step_fused_ct<float>(Fields<const float>, Fields<float>, float*, const Grid&,
-                                          const StepParams<float>&, hipStream_t, int, const SrcParams<float>*, bool,
+                                          const StepParams<float>&, hipStream_t, int, const SrcParams<float>*, int,
                                           bool*);
 template bool launch_step_fused_ct<double>(Fields<const double>, Fields<double>, double*, const Grid&,
-                                           const StepParams<double>&, hipStream_t, int, const SrcParams<double>*, bool,
+                                           const StepParams<double>&, hipStream_t, int, const SrcParams<double>*, int,
                                            bool*);
 
 template bool launch_step_fused<float>(Fields<const float>, Fields<float>, const Grid&, const StepParams<float>&,

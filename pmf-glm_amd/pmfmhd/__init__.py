@@ -386,7 +386,8 @@ def set_ct_kernel(s: MHDState, per_cell: bool):
 def set_ct_workspace(s: MHDState, fill: bool):
     """Fused CT step: write workspace slots 3-14 and form the edge EMFs in a separate pass,
     as the reference's step does (fill=True), or form the edge EMFs in the step kernel and
-    leave slots 3-14 alone (the default); cells, faces and edge EMFs are equal either way."""
+    leave slots 3-14 alone (fill=False); cells, faces and edge EMFs are equal either way. By
+    default PLM steps leave the slots alone and PPM steps write them."""
     check(lib().pmf_set_ct_workspace(s.handle, 1 if fill else 0))
 
 

@@ -158,9 +158,10 @@ int pmf_set_chunk(pmf_state* s, int32_t zc);
 int pmf_autotune(pmf_state* s, int32_t reps, int32_t* zc_out, double* ms_out);
 /* Kernel of the :ref step. By default a state's :ref steps (constrained transport and
  * GLM; plain, drag and radiation steps alike) run on the fused z-marching kernel, which
- * solves every face once with the :ref algorithm (integrator_ref.jl:83-139, 222-258);
- * per_cell != 0 selects the per-cell kernel of integrator_ref.jl:189-220 instead. No
- * counterpart in the reference (one kernel there); results agree to rounding. */
+ * solves every face once with the :ref algorithm (integrator_ref.jl:83-139, 222-258); GLM
+ * steps on grids so thin that the per-cell kernel of integrator_ref.jl:189-220 is faster run
+ * on that one. per_cell != 0 selects the per-cell kernel for all of them. No counterpart in
+ * the reference (one kernel there); results agree to rounding. */
 int pmf_set_ct_kernel(pmf_state* s, int32_t per_cell);
 /* Workspace slots of the fused CT step. The reference's step writes every face's mass and
  * transverse-field fluxes and every cell's EMF to slots 3-14 of the CTState buffer, and

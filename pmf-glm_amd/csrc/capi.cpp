@@ -44,17 +44,14 @@ double smax_device(pmf_state* s) {
   return s->hval[0];
 }
 
-// Whether the :ref integrator's GLM steps run on the fused kernel: the same scheme (PLM the
-// same bits, PPM to rounding) with every face solved and every cell predicted once. It was
-// the faster one on every grid measured: 8^3 34 -> 13.5 us, 32^3 35 -> 14, 128^3 577 -> 110,
-// 200x125x83 MonCen with boundaries 519 -> 113 (float); 160^3 float64 2731 -> 572; 128^3 drag
-// and radiation steps 461-1095 -> 162-231 (float), 1176-1598 -> 451-562 (float64). The per-cell
-// kernel keeps reflecting axes of one cell, grids whose partial maxima do
-// not fit the workspace, and pmf_set_ct_kernel.
-bool ref_on_fused(const pmf_state* s) {
+// Whether a GLM step of the :ref integrator runs on the fused kernel: the same scheme (PLM the
+// same bits, PPM to rounding) with every face solved and every cell predicted once. The per-cell
+// kernel keeps the thin grids on which it is faster (ref_step_fused), reflecting axes of one cell,
+// grids whose partial maxima do not fit the workspace, and pmf_set_ct_kernel.
+bool ref_on_fused(const pmf_state* s, int recon, int rsolve, bool src) {
   const bool f64 = s->p.precision == PMF_F64;
-  return !s->percell && s->p.solver == PMF_SOLVER_GLM &&
-         fused_supported(s->G, s->p.precision, s->p.recon, s->p.riemann) && fused_blocks(s->G, f64, s->zc) <= s->nred;
+  return !s->percell && s->p.solver == PMF_SOLVER_GLM && fused_supported(s->G, s->p.precision, recon, rsolve) &&
+         fused_blocks(s->G, f64, s->zc) <= s->nred && ref_step_fused(s->G, f64, recon, src, s->zc);
 }
 
 // One step from fields `in` into fields `out` (integrator_ref.jl:69-172 / the cube launch),
@@ -74,7 +71,7 @@ bool step_fields(pmf_state* s, Fields<const T> in, Fields<T> out, T* ctp, double
                 "integrators)");
   if (!ct && !(ch > 0.0)) throw Error("step! needs the GLM cleaning speed `ch` (GLM states)");
   if (ct && !ctp) throw Error("ct_update! needs a CT state");
-  const bool fused = integrator == PMF_INTEGRATOR_CUBE || ref_on_fused(s);
+  const bool fused = integrator == PMF_INTEGRATOR_CUBE || ref_on_fused(s, s->p.recon, s->p.riemann, false);
   if (fused) {
     if (!fused_supported(s->G, s->p.precision, s->p.recon, s->p.riemann))
       throw Error("step_cube!: the fused kernel needs every axis at least one cell and reflecting axes two "
@@ -196,7 +193,7 @@ bool step_fields_src(pmf_state* s, Fields<const T> in, Fields<T> out, T* ctp, do
   } else if (a.flags & PMF_SRC_GLOBAL_FALLBACK) {
     P.rsolve = RS_LLF;
   }
-  const bool fused = cube || ref_on_fused(s);
+  const bool fused = cube || ref_on_fused(s, P.recon, P.rsolve, true);
   if (fused) {
     if (!fused_supported(s->G, s->p.precision, P.recon, P.rsolve))
       throw Error(std::string(what) + ": the fused kernel needs every axis at least one cell and reflecting axes two "

@@ -40,6 +40,9 @@ void launch_step_params(const double* dsmax, const double* red, int64_t nb, cons
                         StepParams<T>* Pd, double* clock, double cfl, double glm_ch_fac, double glm_cr, double dx,
                         int reset, hipStream_t st);
 bool fused_supported(const Grid& G, int precision, int recon, int rsolve);
+// Whether a :ref GLM step (src: with drag / radiation sources) is faster on the fused kernel with
+// z chunks of zc planes than on the per-cell kernel.
+bool ref_step_fused(const Grid& G, bool f64, int recon, bool src, int zc);
 bool all_periodic(const Grid& G);
 bool surrogate_grid(const Grid& G);
 // The fused CT step (constrained-transport states, the :ref algorithm with each face

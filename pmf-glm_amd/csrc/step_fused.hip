@@ -22,6 +22,7 @@
 // once, and the global state is read once and written once per step. Workgroups are
 // remapped so that consecutive tiles land on the same XCD (and its L2), which then
 // serves the halo re-reads.
+#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
@@ -1233,6 +1234,29 @@ int fused_chunk(const Grid& G, bool f64) { return chunk_of(G, 0, f64); }
 int64_t fused_blocks(const Grid& G, bool f64, int zc) {
   FusedGeom g = fused_geom(G, chunk_of(G, zc, f64));
   return (int64_t)g.ntx * g.nty * g.nchunks;
+}
+
+// Whether a :ref GLM step is faster on the fused kernel than on the per-cell one, which solves
+// six faces and predicts seven cells for every cell, but only for cells that exist: on a grid
+// that is thin in x or y most columns of the fused kernel's 16 x 12 tiles are empty, and a long
+// thin one marches many planes for few cells ((1, 1, 65536) float MonCen: 411 us against 29,
+// (1, 2048, 2048): 2503 against 940). Both times are estimated in us. Fused: 5, and per unit of
+// fused_cost 3.4 (float; with sources 4.2), 5.3 (float64 PLM, two workgroups a CU) or 6.2 (float64
+// PPM, one; with sources 6.9), a seventh more where rows shorter than a tile's break up the loads.
+// Per-cell: 29 (float PLM; PPM 38, sources 33) or 42 (float64; sources 37) for a round of two
+// (float64: one) blocks of 256 cells a CU. Over 318 combinations of 53 grids, both precisions, PLM,
+// PPM and drag the estimate takes the slower kernel three times, by at most 8%. Where the fused one
+// wins (us, per-cell -> fused): 8^3 28.6 -> 15.9, (4096, 1, 1) 29 -> 16, (256, 256, 1) 31 -> 18,
+// (512, 512, 3) 198 -> 61, 200x125x83 with boundaries 519 -> 108; float64 (256, 256, 1) 48 -> 29,
+// (2048, 2048, 1) 2648 -> 920.
+bool ref_step_fused(const Grid& G, bool f64, int recon, bool src, int zc) {
+  const FusedGeom g = fused_geom(G, chunk_of(G, zc, f64));
+  const int places = !f64 ? 3 : recon == RECON_PPM || src ? 1 : 2;
+  const double unit = (places == 3 ? (src ? 4.2 : 3.4) : places == 2 ? 5.3 : src ? 6.9 : 6.2) * (G.nx < TX ? 1.15 : 1.0);
+  const double fused = 5.0 + unit * fused_cost((int64_t)g.ntx * g.nty * g.nchunks, g.zc, places);
+  const double round = f64 ? (src ? 37.0 : 42.0) : src ? 33.0 : recon == RECON_PPM ? 38.0 : 29.0;
+  const double rounds = double(G.nc) / (256.0 * (f64 ? 1 : 2) * device_cus());
+  return fused < round * std::max(1.0, rounds + 0.25);
 }
 
 template <class T>

@@ -379,7 +379,8 @@ def set_chunk(s: MHDState, zc: int):
 
 def set_ct_kernel(s: MHDState, per_cell: bool):
     """:ref steps (CT and GLM) on the per-cell kernel (True) or on the fused kernel that
-    solves every face once (False, the default)."""
+    solves every face once (False, the default; GLM steps on thin grids stay on the per-cell
+    kernel where that is faster)."""
     check(lib().pmf_set_ct_kernel(s.handle, 1 if per_cell else 0))
 
 

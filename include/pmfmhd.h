@@ -107,8 +107,9 @@ int pmf_max_wavespeed_of(pmf_state* s, const void* const* U, double* smax);
  * device, kept until the process ends: grids whose fused step needs more than 2^18
  * per-workgroup partial slots (about 1.6e9 cells at the built-in chunk) are refused with an
  * error naming pmf_step_into. smax_dev (optional, a caller device double) receives the
- * CFL speed of the output fields (max_wavespeed!, timestep.jl:17-23). Calls that overlap
- * on one device share the workspace and race; calls on one stream are ordered. */
+ * CFL speed of the output fields (max_wavespeed!, timestep.jl:17-23). Only calls with
+ * smax_dev use the workspace: those that overlap on one device share it and race; calls on
+ * one stream are ordered. */
 int pmf_step_into_static(const pmf_params* p, const void* const* U, void* const* O, void* ct, double dt, double ch,
                          double decay, int32_t integrator, void* hip_stream, double* smax_dev);
 /* evolve! (driver.jl:48-71) without a callback: CFL steps until t >= tfinal(1-1e-9),

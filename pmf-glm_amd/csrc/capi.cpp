@@ -57,11 +57,13 @@ bool ref_on_fused(const pmf_state* s, int recon, int rsolve, bool src) {
 // One step from fields `in` into fields `out` (integrator_ref.jl:69-172 / the cube launch),
 // then ct_update! on `out` for CT states (ct.jl:158-173). No swap. Returns whether the new
 // state's CFL speed was folded into dval[0] and hval[0]; with fold = false (the caller's
-// arrays, whose speed the state does not keep) that reduction is left out.
+// arrays, whose speed the state does not keep) that reduction is left out, and nothing is written
+// to the workspace, so that calls on several streams do not meet there.
 template <class T>
 bool step_fields(pmf_state* s, Fields<const T> in, Fields<T> out, T* ctp, double dt, double ch, double decay,
                  int integrator, bool fold) {
   double* const dsmax = fold ? s->dval : nullptr;
+  double* const red = fold ? s->red : nullptr;
   const bool ct = s->p.solver == PMF_SOLVER_CT;
   bool edges = false;  // CT: the step kernel formed the edge EMFs
   if (integrator != PMF_INTEGRATOR_REF && integrator != PMF_INTEGRATOR_CUBE)
@@ -79,7 +81,7 @@ bool step_fields(pmf_state* s, Fields<const T> in, Fields<T> out, T* ctp, double
                   ")");
     mark(s);
     bool done =
-        launch_step_fused<T>(in, out, s->G, make_params<T>(s, dt, ch, decay), s->red, dsmax, s->st, s->zc, nullptr,
+        launch_step_fused<T>(in, out, s->G, make_params<T>(s, dt, ch, decay), red, dsmax, s->st, s->zc, nullptr,
                              nullptr, s->hval);
     mark(s);
     if (!done) throw Error("step_cube!: fused kernel unavailable for this configuration");
@@ -139,6 +141,7 @@ template <class T>
 bool step_fields_src(pmf_state* s, Fields<const T> in, Fields<T> out, T* ctp, double dt, double ch, double decay,
                      int integrator, const SourceCall& a, bool fold) {
   double* const dsmax = fold ? s->dval : nullptr;
+  double* const red = fold ? s->red : nullptr;
   const bool ct = s->p.solver == PMF_SOLVER_CT;
   const bool cube = integrator == PMF_INTEGRATOR_CUBE;
   const char* what = a.radiation ? (cube ? "step_cube_radiation!" : "step_ref_radiation!")
@@ -200,7 +203,7 @@ bool step_fields_src(pmf_state* s, Fields<const T> in, Fields<T> out, T* ctp, do
                                       "(got " + std::to_string(s->p.nx) + "x" + std::to_string(s->p.ny) + "x" +
                   std::to_string(s->p.nz) + ")");
     mark(s);
-    bool done = launch_step_fused<T>(in, out, s->G, P, s->red, dsmax, s->st, s->zc, &S, nullptr, s->hval);
+    bool done = launch_step_fused<T>(in, out, s->G, P, red, dsmax, s->st, s->zc, &S, nullptr, s->hval);
     mark(s);
     if (!done) throw Error(std::string(what) + ": fused kernel unavailable for this configuration");
   } else if (ct && !s->percell && S.check != CHECK_MASKED && S.check != CHECK_GLOBAL &&
@@ -857,8 +860,8 @@ int pmf_max_wavespeed_of(pmf_state* s, const void* const* U, double* smax) {
 // capture, serving loops, hosts that forbid it): no pmf_state, the caller's stream, and
 // the kernels' workspace (per-workgroup partial maxima of the CFL fold, then the device
 // scalars) in one file-scope device array. Every block writes its own partial slot before
-// the final fold reads it, so nothing in the array has to start at zero. Calls that
-// overlap on one device share the array and race.
+// the final fold reads it, so nothing in the array has to start at zero. Only calls that ask
+// for the speed use the array: those that overlap on one device race.
 namespace {
 constexpr int64_t kStaticPartials = int64_t(1) << 18;  // doubles: per-workgroup partials
 constexpr int64_t kStaticScalars = 64;                 // doubles: [0] = CFL speed of the output

@@ -18,7 +18,7 @@ void launch_step_ref(Fields<const T> U, Fields<T> O, T* ctp, const Grid& G, cons
                      hipStream_t st, const SrcParams<T>* S = nullptr);
 
 // Fused tiled step (periodic GLM). Writes per-block CFL maxima of the new state into
-// red (one double per block) and, unless dsmax is null, the final max into *dsmax and, if
+// red (one double per block), unless that is null, and, unless dsmax is null, the final max into *dsmax and, if
 // given, *hsmax (pinned host memory). Returns false when the grid shape is not supported by
 // the fused kernel.
 // zc: planes per z chunk (0 = the built-in choice); src: drag / radiation source terms

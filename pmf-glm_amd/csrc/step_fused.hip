@@ -963,8 +963,8 @@ __device__ __forceinline__ void step_fused_body(const Fields<const T>& U, const 
   const T smax =
       fused_item<T, RECON, RS, SURR, SRC, NARROW, false, BCG, false, AHEAD>(U, O, g, P, w, lds, sW, thr, smooth_count,
                                                                            src, q);
-  // fold the workgroup's CFL maximum (timestep.jl:8-12 on the new state)
-  block_store_max(smax, sMax, red + blockIdx.x);
+  // fold the workgroup's CFL maximum (timestep.jl:8-12 on the new state), if the caller wants it
+  if (red) block_store_max(smax, sMax, red + blockIdx.x);
   if constexpr (SURR) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) smooth_count += __shfl_xor(smooth_count, o, 64);

@@ -248,6 +248,11 @@ __device__ __forceinline__ void hancock_plm(const T* m0, const T* dRx, const T* 
 __device__ __forceinline__ float med3z(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, 0.f); }
 __device__ __forceinline__ double med3z(double a, double b) { return dmax(dmin(a, b), dmin(dmax(a, b), 0.0)); }
 
+// NaN if c, else x (the upper half of the double decides, so one select does).
+__device__ __forceinline__ double nan_if(bool c, double x) {
+  return __hiloint2double(c ? 0x7ff80000 : __double2hiint(x), __double2loint(x));
+}
+
 // PLM face offsets (dL, dR) from the one-sided differences dl = q0 - qm and dr = qp - q0
 // (glm_physics.jl:47-59), for offsets<RECON> and for callers that already hold a
 // difference (the fused step carries each column's z difference from one plane to the
@@ -282,6 +287,12 @@ template <int RECON, class T> __device__ __forceinline__ void offsets(T qm, T q0
     T a = slope + curve, b = slope - curve;
     dR = med3z(a, T(2) * b);
     dL = -med3z(b, T(2) * a);
+    // the float64 medians drop a NaN; the cell's neighbours are to see it as it was
+    if constexpr (sizeof(T) == 8) {
+      const bool nan = __builtin_isunordered(a, b);
+      dR = nan_if(nan, dR);
+      dL = nan_if(nan, dL);
+    }
   } else {
     offsets_diff<RECON>(q0 - qm, qp - q0, dL, dR);
   }

@@ -155,7 +155,8 @@ int pmf_set_chunk(pmf_state* s, int32_t zc);
  * chunks of 4..128 planes (reps launches each, writing only the scratch fields and, for
  * CT, the per-step workspace slots) and keeps the fastest; returns it and its time per
  * step. Small grids whose built-in choice is shorter than 4 planes keep that one if it is
- * faster; the depth returned is then the fastest of 4..128. */
+ * faster still; the depth and time returned are always those of the fastest of 4..128, so
+ * that pmf_set_chunk with that depth gives that time. */
 int pmf_autotune(pmf_state* s, int32_t reps, int32_t* zc_out, double* ms_out);
 /* Kernel of the :ref step. By default a state's :ref steps (constrained transport and
  * GLM; plain, drag and radiation steps alike) run on the fused z-marching kernel, which

@@ -617,7 +617,7 @@ int pmf_autotune(pmf_state* s, int32_t reps, int32_t* zc_out, double* ms_out) {
     double best = 1e300, best_set = 1e300;
     try {
       // the built-in choice (0) too, where it is shorter than any depth a caller may set: it is
-      // kept if it is the fastest, and the depth returned is then the fastest settable one
+      // kept if it is the fastest; the depth and time returned are those of the fastest settable one
       const int first = fused_chunk(s->G, s->p.precision == PMF_F64) < kMinChunk ? 0 : 4;
       for (int zc : {0, 4, 8, 12, 16, 24, 32, 48, 64, 96, 128}) {
         if (zc < first) continue;
@@ -669,7 +669,7 @@ int pmf_autotune(pmf_state* s, int32_t reps, int32_t* zc_out, double* ms_out) {
     s->zc = keep_zc;
     s->smax_valid = false;  // dval now holds the speed of the scratch fields
     if (zc_out) *zc_out = best_zc;
-    if (ms_out) *ms_out = best;
+    if (ms_out) *ms_out = best_set;
   });
 }
 

@@ -1062,14 +1062,14 @@ template <class T> inline bool narrow_fields(int64_t nc) {
   return (uint64_t)nc * sizeof(T) < (1ull << 32);
 }
 
-// Maximum of red[0 .. nb), NaN if one is; every thread of the one block of 1024 gets it. Eight
+// Maximum of red[0 .. nb), NaN if one is; every thread of the one block of TH gets it. Eight
 // loads in flight a thread: with 256 threads and one load at a time the 22016 partials of a
 // 512^3 step took 37 us; the 2816 of 256^3, 5.0.
-__device__ __forceinline__ double fold_max(const double* __restrict__ red, int nb, double* sh) {
+template <int TH> __device__ __forceinline__ double fold_max(const double* __restrict__ red, int nb, double* sh) {
   double m[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  for (int b = threadIdx.x; b < nb; b += 8 * 1024) {
+  for (int b = threadIdx.x; b < nb; b += 8 * TH) {
 #pragma unroll
-    for (int k = 0; k < 8; ++k) m[k] = nanmax(m[k], red[min(b + k * 1024, nb - 1)]);
+    for (int k = 0; k < 8; ++k) m[k] = nanmax(m[k], red[min(b + k * TH, nb - 1)]);
   }
 #pragma unroll
   for (int k = 4; k > 0; k >>= 1)
@@ -1080,22 +1080,29 @@ __device__ __forceinline__ double fold_max(const double* __restrict__ red, int n
   __syncthreads();
   double r = sh[0];
 #pragma unroll
-  for (int k = 1; k < 16; ++k) r = nanmax(r, sh[k]);
+  for (int k = 1; k < TH / 64; ++k) r = nanmax(r, sh[k]);
   return r;
 }
 
-__global__ __launch_bounds__(1024) void k_fold_max_flat(const double* __restrict__ red, int nb, double* __restrict__ out,
-                                                        double* __restrict__ hout) {
-  __shared__ double sh[16];
-  const double r = fold_max(red, nb, sh);
+template <int TH>
+__global__ __launch_bounds__(TH) void k_fold_max_flat(const double* __restrict__ red, int nb, double* __restrict__ out,
+                                                      double* __restrict__ hout) {
+  __shared__ double sh[TH / 64];
+  const double r = fold_max<TH>(red, nb, sh);
   if (threadIdx.x == 0) {
     out[0] = r;
     if (hout) hout[0] = r;
   }
 }
 
+// 256 threads while they take all partials with one round of loads: sixteen waves to start and to
+// wait for cost 0.6 to 1.1 us more (queued step, LLF: (256, 256, 1) 15.8 us with 1024 threads,
+// 15.0 with 256; 64^3 25.3, 24.5; (512, 512, 3), 1376 partials, 52.5, 51.3).
 void launch_fold_max(const double* red, int64_t nb, double* dsmax, double* hsmax, hipStream_t st) {
-  hipLaunchKernelGGL(k_fold_max_flat, dim3(1), dim3(1024), 0, st, red, (int)nb, dsmax, hsmax);
+  if (nb <= 8 * 256)
+    hipLaunchKernelGGL(k_fold_max_flat<256>, dim3(1), dim3(256), 0, st, red, (int)nb, dsmax, hsmax);
+  else
+    hipLaunchKernelGGL(k_fold_max_flat<1024>, dim3(1), dim3(1024), 0, st, red, (int)nb, dsmax, hsmax);
 }
 
 // The device-side CFL stage of pmf_advance: evolve!'s step rule (driver.jl:48-71) from
@@ -1110,7 +1117,7 @@ __global__ __launch_bounds__(1024) void k_step_params(const double* __restrict__
                                                       double dx, int reset) {
 #pragma clang fp contract(off)
   __shared__ double sh[16];
-  const double sm = nb > 0 ? fold_max(red, nb, sh) : dsmax[0];
+  const double sm = nb > 0 ? fold_max<1024>(red, nb, sh) : dsmax[0];
   if (threadIdx.x != 0) return;
   double dtf, ch, decay;
   if constexpr (sizeof(T) == 8) {

@@ -83,10 +83,10 @@ int pmf_compute_dt(pmf_state* s, double cfl, double* dt, double* smax);
 /* step_ref! / step_cube! (integrator_ref.jl:210-220, integrator_cube.jl:455-463): one
  * MUSCL-Hancock step of size dt with GLM speed ch and psi factor decay, written to
  * scratch and swapped in; CT states also run ct_update! (ct.jl:158-173) and ignore ch
- * and decay. integrator: PMF_INTEGRATOR_REF (per-cell recompute) or
- * PMF_INTEGRATOR_CUBE (fused tiled kernel; GLM only; any grid shape and boundary codes,
- * where the reference's needs a cubic N % 4 == 0 grid; a reflecting axis needs two
- * cells). */
+ * and decay. integrator: PMF_INTEGRATOR_REF (any grid and solver; the fused kernel or the
+ * per-cell one, see pmf_set_ct_kernel) or PMF_INTEGRATOR_CUBE (always the fused tiled kernel;
+ * GLM only; any grid shape and boundary codes, where the reference's needs a cubic N % 4 == 0
+ * grid; a reflecting axis needs two cells). */
 int pmf_step_raw(pmf_state* s, double dt, double ch, double decay, int32_t integrator);
 /* step! (driver.jl:20-37): decay = exp(-glm_cr*ch*dt/dx) in the state's precision. */
 int pmf_step(pmf_state* s, double dt, double ch, double glm_cr, int32_t integrator);

@@ -921,10 +921,12 @@ __device__ __forceinline__ void block_store_max(T smax, T* sMax, double* out) {
 }
 
 // Three waves per SIMD (168 VGPRs; three 38 KB workgroups then share a CU's LDS) for
-// every plain float variant and the PLM source variants. PLM fits the plain step without
-// spilling, the PLM source variants (drag, radiation) among them; PPM keeps both edge offsets
-// of each direction live and is still faster at three waves than at two. The PPM source
-// variants would spill 44 and keep the compiler's default (two waves).
+// every plain float variant and the PLM source variants. PLM fits without spilling, but for the
+// source instances that issue their loads ahead: those spill 5 to 7 registers (24 to 32 bytes of
+// scratch a lane) and are 5% faster than the ones that do not (loads_ahead). PPM keeps both edge
+// offsets of each direction live and is still faster at three waves than at two. The PPM source
+// variants take 166 to 172 registers uncapped, without spills: with 32-bit offsets on periodic
+// grids three waves, most of the others two.
 template <class T, int RECON, int RS, bool SURR, bool SRC>
 constexpr bool fused_three_waves() {
   return sizeof(T) == 4 && !SURR && !(SRC && RECON == RECON_PPM);
@@ -1203,8 +1205,11 @@ bool surrogate_grid(const Grid& G) { return all_periodic(G) && G.nx % TX == 0 &&
 // last, partly filled one. Chunks past 32 planes repeat under 6% and measured no faster (256^3
 // 32: 790 us, 64: 876; 512^3 5.93 and 6.06 ms).
 // Measured (minmod, step and fold, the earlier rule's choice -> this one's): 16^3 23.7 -> 12.9
-// us (4 planes -> 1), 32^3 23.7 -> 13.6 (1), 64^3 31.4 -> 28.6 (2), 96^3 64 -> 55 (6); 128^3 (16)
-// and 256^3 (32) as before.
+// us (4 planes -> 1), 32^3 23.7 -> 13.6 (1), 64^3 31.4 -> 28.6 (2), 96^3 62.3 -> 52 (6). 128^3 (16
+// planes, 109 us), 192^3 (24, 323) and 256^3 (32, 754; 750 at 16) take the best depth or one within
+// 1% of it. Not so 112^3 (16, 92.6; 85.7 at 4, the earlier choice), 160^3 (32, 210; 200 at 8, the
+// earlier choice) and 250^3 (28, 740; 726 at 16). float64 PPM and source steps, of which a CU holds
+// one workgroup, get the length for two.
 double fused_cost(int64_t groups, int zc, int slots) {
   static const double kShare[2][4] = {{0, 1.0, 1.45, 1.45}, {0, 1.0, 1.19, 1.54}};
   const double* share = kShare[slots >= 3];

@@ -762,7 +762,8 @@ int pmf_surrogate_train(pmf_surrogate* n, int32_t batch, int32_t steps, double l
     if (!n || n->n < 1) throw Error("the dataset is empty");
     if (batch < 1 || steps < 0) throw Error("bad arguments");
     // Two launches a step and no wait between steps: the losses stay on the device until the
-    // end. Batch 8192: 6.9 ms a step layer by layer, 27 us now (4096: 20, 1024: 14.5).
+    // end. Batch 8192: 6.9 ms a step layer by layer, now 27 us of 128 or more in a call, 31 of eight
+    // (4096: 20 and 24, 1024: 15 and 19).
     grow(n->dloss, n->loss_steps, std::max<int64_t>(steps, 1), 1);
     Adam a;
     a.on = 1;

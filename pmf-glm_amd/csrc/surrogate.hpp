@@ -120,10 +120,6 @@ __device__ __forceinline__ float gelu_grad(float z) {
 __device__ __forceinline__ unsigned short bf16_bits(float f) {
   return __builtin_bit_cast(unsigned short, (__bf16)f);
 }
-__device__ __forceinline__ float bf16_round(float f) {
-  unsigned u = (unsigned)bf16_bits(f) << 16;
-  return __builtin_bit_cast(float, u);
-}
 
 }  // namespace pmf
 

@@ -530,12 +530,14 @@ struct pmf_surrogate {
 
 namespace {
 
+// At least `want` elements of `each` T. The old buffer goes only when the new one is there: if the
+// device has no room, p stays what it was (later calls rely on one loss).
 template <class T> void grow(T*& p, int64_t& have, int64_t want, int64_t each) {
   if (want <= have) return;
+  T* q = nullptr;
+  hip_check(hipMalloc(&q, sizeof(T) * each * want), "hipMalloc");
   (void)hipFree(p);
-  p = nullptr;
-  have = 0;
-  hip_check(hipMalloc(&p, sizeof(T) * each * want), "hipMalloc");
+  p = q;
   have = want;
 }
 

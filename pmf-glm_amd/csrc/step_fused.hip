@@ -1257,7 +1257,7 @@ int64_t fused_blocks(const Grid& G, bool f64, int zc) {
 // PPM, one; with sources 6.9), a seventh more where rows shorter than a tile's break up the loads.
 // Per-cell: 29 (float PLM; PPM 38, sources 33) or 42 (float64; sources 37) for a round of two
 // (float64: one) blocks of 256 cells a CU. Over 318 combinations of 53 grids, both precisions, PLM,
-// PPM and drag the estimate takes the slower kernel three times, by at most 8%. Where the fused one
+// PPM and drag the estimate takes the slower kernel three times, by at most 9%. Where the fused one
 // wins (us, per-cell -> fused): 8^3 28.6 -> 15.9, (4096, 1, 1) 29 -> 16, (256, 256, 1) 31 -> 18,
 // (512, 512, 3) 198 -> 61, 200x125x83 with boundaries 519 -> 108; float64 (256, 256, 1) 48 -> 29,
 // (2048, 2048, 1) 2648 -> 920.
